@@ -115,7 +115,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
     for (int r = blockIdx.x; r < a.nreal; r += gridDim.x) {
         if (tid < kStatCount)
             s_stat[tid] = 0;
-        int ok = 1;
+        int ok = min(plain_origin(a.xo), plain_origin(a.yo));
         for (int i = tid; i < a.nwells; i += blockDim.x) {
             Well64 wl;
             wl.x = a.wells_xy[2 * i];
@@ -123,15 +123,17 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
             wl.nq = -a.q[(int64_t)r * a.nwells + i];
             wl.pad = 0.0;
             s_wells[i] = wl;
-            ok &= plain_coord(wl.x) && plain_coord(wl.y) && plain_strength(wl.nq);
+            ok = min(ok, plain_well(wl));
         }
         if (raster)
             ch.begin(a);
         if (tid == 0)
             s_next = blockDim.x;
-        const bool plain = __syncthreads_and(ok) != 0;
+        const int plain = __syncthreads_and(ok >= kPlainBelow) ? kPlainBelow
+                          : __syncthreads_and(ok >= kPlainCoord) ? kPlainCoord
+                                                                 : kPlainNever;
 
-        const Field64 f = make_field(a, r, s_wells, plain);
+        const Field64 f = make_field(a, r, s_wells, __builtin_amdgcn_readfirstlane(plain));
         unsigned long long n_att = 0, n_acc = 0, n_esc = 0, n_cand = 0;
         unsigned long long n_st[4] = {0, 0, 0, 0};
 
@@ -153,7 +155,8 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
                     a.verts[2 * (k * a.vcap)] = xs;
                     a.verts[2 * (k * a.vcap) + 1] = ys;
                 }
-                live = dp5_start<kConfined>(f, I, s, xs, ys);
+                open64(s, I, xs, ys);
+                live = dp5_start<kConfined>(f, I, s);
                 ended = !live;
             } else {
                 double ox, oy;

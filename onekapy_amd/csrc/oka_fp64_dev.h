@@ -49,39 +49,14 @@ struct __align__(16) Well64 {
 struct Field64 {
     const Well64 *w;
     int nw;
-    bool plain;          // every well passes plain_coord / plain_strength
+    int plain;           // kPlain*: when the short division sequences apply
     double xo, yo;
     double A, B, C, D, E, F;
     double A2, B2;       // 2.0*A, 2.0*B (exact)
     double K, bt, bn;    // conductivity, thickness, thickness*porosity
+    double rbn;          // recip_plain(bn)
     double por, half_kb2;
 };
-
-__device__ __forceinline__ Field64 make_field(const TraceArgs &a, int r, const Well64 *w,
-                                              bool plain)
-{
-    Field64 f;
-    f.w = w;
-    f.plain = plain;
-    f.nw = a.nwells;
-    f.xo = a.xo;
-    f.yo = a.yo;
-    const double *c = a.coef + 6 * (int64_t)r;
-    f.A = c[0];
-    f.B = c[1];
-    f.C = c[2];
-    f.D = c[3];
-    f.E = c[4];
-    f.F = c[5];
-    f.A2 = 2.0 * f.A;
-    f.B2 = 2.0 * f.B;
-    f.K = a.K[r];
-    f.bt = a.b[r];
-    f.por = a.n[r];
-    f.bn = f.bt * f.por;
-    f.half_kb2 = (0.5 * f.K) * (f.bt * f.bt);
-    return f;
-}
 
 // a1 / b and a2 / b, each correctly rounded (IEEE division, as numpy's).
 // gfx950 has no division instruction; the compiler expands every FP64 `/`
@@ -115,20 +90,36 @@ __device__ __forceinline__ void div_pair(double a1, double a2, double b, double 
         __builtin_amdgcn_div_fmas(fma(-d, m2, n2), r, m2, s2), b, a2);
 }
 
-// a1 / b and a2 / b, each correctly rounded, for operands that need none of
-// div_scale's scalings (see plain_coord): then div_scale returns its operand
-// unchanged and div_fmas is a plain fma, so the sequence above reduces to
-// this one with the same bits.  div_fixup stays: it gives a zero numerator
-// its signed zero and 0/0 its NaN, exactly as in the full sequence.
-__device__ __forceinline__ void div_pair_plain(double a1, double a2, double b, double &q1,
-                                               double &q2)
+// 1 / b for a divisor that needs no scaling (see plain_coord): the hardware
+// estimate r0 (relative error e0 below 2^-23, measured 2^-24.3 at most over
+// 4e9 divisors) and one third-order step, r0 (1 + e0 + e0^2), whose error
+// before its rounding is e0^3 < 2^-69.  One instruction less than two Newton
+// steps.  With quot_plain a well term takes 21 VALU instructions instead of 24
+// (the tracer is bound by their issue): 10^4 x 1000 particles of a 25-well
+// site 149.8 -> 132.7 ms, with the regional quotient's shared reciprocal.
+__device__ __forceinline__ double recip_plain(double b)
 {
-    double r = __builtin_amdgcn_rcp(b);
-    r = fma(r, fma(-b, r, 1.0), r);
-    r = fma(r, fma(-b, r, 1.0), r);
-    const double m1 = a1 * r, m2 = a2 * r;
-    q1 = __builtin_amdgcn_div_fixup(fma(fma(-b, m1, a1), r, m1), b, a1);
-    q2 = __builtin_amdgcn_div_fixup(fma(fma(-b, m2, a2), r, m2), b, a2);
+    const double r0 = __builtin_amdgcn_rcp(b);
+    const double e = fma(-b, r0, 1.0);
+    return fma(r0, fma(e, e, e), r0);
+}
+
+// a / b correctly rounded from r = recip_plain(b), for operands that need no
+// scaling.  With |r b - 1| <= (1 + 2^-16) 2^-54 m (m in [1, 2) the mantissa of
+// b), q0 = RN(a r) is one of the two doubles around any rounding boundary
+// next to a / b, the residual a - b q0 is exact, and q0 + residual r lies
+// within 2^-107 m (1 + 2^-16) (times the exponent of the quotient) of a / b.
+// A quotient differs from a rounding boundary by at least 2^-105 / m, so the
+// final rounding is that of a / b for every m < 2 - 2^-16 (above it only
+// numerators within 2^-53 of the worst case could differ, as in the
+// compiler's own sequence at m = 2 - 2^-52).  The residual is formed negated,
+// b q0 - a, so that a zero numerator keeps its sign through the sum
+// (-(+0) r + (-0) = -0) and no div_fixup is needed.  0 / 0 gives NaN: r0 is
+// infinite and e0 NaN.
+__device__ __forceinline__ double quot_plain(double a, double b, double r)
+{
+    const double q0 = a * r;
+    return fma(-fma(b, q0, -a), r, q0);
 }
 
 // The well terms' divisions (-q dx) / r2 and (-q dy) / r2 need no scaling
@@ -140,6 +131,9 @@ __device__ __forceinline__ void div_pair_plain(double a1, double a2, double b, d
 // is subnormal -- none of div_scale's conditions (tiny or huge denominator,
 // exponent gap >= 768, subnormal quotient, numerator exponent <= 53) holds.
 // r2 = 0 implies zero numerators: 0 / 0 gives NaN in both sequences.
+// A point coordinate below 2^-200 is as good as 0 where every well's (and the
+// origin's) coordinate is at least 2^-200 in magnitude: their difference is
+// then the well's coordinate to within rounding.
 __device__ __forceinline__ bool plain_coord(double v)
 {
     const double a = fabs(v);
@@ -150,6 +144,75 @@ __device__ __forceinline__ bool plain_strength(double nq)
 {
     const double a = fabs(nq);
     return a == 0.0 || (a >= 0x1p-100 && a <= 0x1p100);
+}
+
+// Field64::plain: the short sequences never; where the point passes
+// plain_coord; or, when no well coordinate is 0, where it is below 2^60.
+enum { kPlainNever = 0, kPlainCoord = 1, kPlainBelow = 2 };
+
+// What well w allows: combine over the wells with min().
+__device__ __forceinline__ int plain_well(const Well64 &w)
+{
+    if (!(plain_coord(w.x) && plain_coord(w.y) && plain_strength(w.nq)))
+        return kPlainNever;
+    return w.x != 0.0 && w.y != 0.0 ? kPlainBelow : kPlainCoord;
+}
+
+// The same of one coordinate of the origin.
+__device__ __forceinline__ int plain_origin(double v)
+{
+    return !plain_coord(v) ? kPlainNever : (v != 0.0 ? kPlainBelow : kPlainCoord);
+}
+
+// Whether the regional part allows the short quotient Q / bn: with these
+// bounds Q is 0 or a multiple of 2^-540, bn and its reciprocal are far from
+// the range's ends, and the residual of quot_plain is exact.
+__device__ __forceinline__ bool plain_term(double c)
+{
+    const double a = fabs(c);
+    return a == 0.0 || (a >= 0x1p-200 && a <= 0x1p100);
+}
+
+__device__ __forceinline__ bool plain_field(const Field64 &f)
+{
+    return plain_term(f.A2) && plain_term(f.B2) && plain_term(f.C) && plain_term(f.D) &&
+           plain_term(f.E) && f.bn >= 0x1p-100 && f.bn <= 0x1p100;
+}
+
+// Whether the point (x, y) allows the short sequences, given that the field
+// does (f.plain != kPlainNever).  NaN coordinates may pass: every sequence
+// gives NaN for them.
+__device__ __forceinline__ bool plain_point(const Field64 &f, double x, double y)
+{
+    return f.plain == kPlainBelow ? fmax(fabs(x), fabs(y)) < 0x1p60
+                                  : plain_coord(x) && plain_coord(y);
+}
+
+__device__ __forceinline__ Field64 make_field(const TraceArgs &a, int r, const Well64 *w,
+                                              int plain)
+{
+    Field64 f;
+    f.w = w;
+    f.nw = a.nwells;
+    f.xo = a.xo;
+    f.yo = a.yo;
+    const double *c = a.coef + 6 * (int64_t)r;
+    f.A = c[0];
+    f.B = c[1];
+    f.C = c[2];
+    f.D = c[3];
+    f.E = c[4];
+    f.F = c[5];
+    f.A2 = 2.0 * f.A;
+    f.B2 = 2.0 * f.B;
+    f.K = a.K[r];
+    f.bt = a.b[r];
+    f.por = a.n[r];
+    f.bn = f.bt * f.por;
+    f.rbn = recip_plain(f.bn);
+    f.half_kb2 = (0.5 * f.K) * (f.bt * f.bt);
+    f.plain = plain_field(f) ? plain : kPlainNever;
+    return f;
 }
 
 // The wells' part of the discharge at (x, y) (model.py:307-313) and, for the
@@ -169,10 +232,13 @@ __device__ __forceinline__ void well_sums(const Field64 &f, double x, double y, 
         const double ddy = y - wl.y;
         const double r2 = ddx * ddx + ddy * ddy;
         double sx, sy;
-        if (kPlain)
-            div_pair_plain(wl.nq * ddx, wl.nq * ddy, r2, sx, sy);
-        else
+        if (kPlain) {
+            const double r = recip_plain(r2);
+            sx = quot_plain(wl.nq * ddx, r2, r);
+            sy = quot_plain(wl.nq * ddy, r2, r);
+        } else {
             div_pair(wl.nq * ddx, wl.nq * ddy, r2, sx, sy);
+        }
         Qx = Qx + sx * kC2Pi;
         Qy = Qy + sy * kC2Pi;
         if (!kConfined)
@@ -181,22 +247,29 @@ __device__ __forceinline__ void well_sums(const Field64 &f, double x, double y, 
 }
 
 // feval(xy) = -V(xy) (stochastic.py:253-260).  Returns false where the
-// reference raises AquiferError (unconfined only).
-template <bool kConfined>
-__device__ __forceinline__ bool feval(const Field64 &f, double x, double y, double &kx, double &ky)
+// reference raises AquiferError (unconfined only).  kPlain uses the short
+// division sequences and clears `ok` when (x, y) does not allow them: the
+// result is then discarded and computed again without kPlain.
+template <bool kConfined, bool kPlain>
+__device__ __forceinline__ bool feval(const Field64 &f, double x, double y, double &kx, double &ky,
+                                      bool &ok)
 {
     const double dx = x - f.xo;
     const double dy = y - f.yo;
     double Qx = -((f.A2 * dx + f.C * dy) + f.D);
     double Qy = -((f.B2 * dy + f.C * dx) + f.E);
     double pw = 0.0;
-    if (f.plain && plain_coord(x) && plain_coord(y))
-        well_sums<kConfined, true>(f, x, y, Qx, Qy, pw);
-    else
-        well_sums<kConfined, false>(f, x, y, Qx, Qy, pw);
+    if (kPlain)
+        ok = ok && plain_point(f, x, y);
+    well_sums<kConfined, kPlain>(f, x, y, Qx, Qy, pw);
+    double vx, vy;
     if (kConfined) {
-        double vx, vy;
-        div_pair(Qx, Qy, f.bn, vx, vy);
+        if (kPlain) {
+            vx = quot_plain(Qx, f.bn, f.rbn);
+            vy = quot_plain(Qy, f.bn, f.rbn);
+        } else {
+            div_pair(Qx, Qy, f.bn, vx, vy);
+        }
         kx = -vx;
         ky = -vy;
         return true;
@@ -213,9 +286,25 @@ __device__ __forceinline__ bool feval(const Field64 &f, double x, double y, doub
     if (head <= 0.0)
         return false;
     const double den = head > f.bt ? f.bn : head * f.por;
-    kx = -(Qx / den);
-    ky = -(Qy / den);
+    div_pair(Qx, Qy, den, vx, vy);
+    kx = -vx;
+    ky = -vy;
     return true;
+}
+
+// One field evaluation of every active lane: with the short sequences, and
+// again without them when the field or any lane's point does not allow them.
+// Both give the same bits where they apply, so one such lane may take its
+// wave along, and the long sequence stays off the usual path.
+template <bool kConfined>
+__device__ __forceinline__ bool eval64(const Field64 &f, double x, double y, double &kx, double &ky)
+{
+    bool ok = f.plain != kPlainNever, wet = false;
+    if (ok)
+        wet = feval<kConfined, true>(f, x, y, kx, ky, ok);
+    if (__ballot(!ok) != 0ull)
+        wet = feval<kConfined, false>(f, x, y, kx, ky, ok);
+    return wet;
 }
 
 struct Integ {
@@ -230,11 +319,8 @@ struct Trace64 {
     int status;
 };
 
-// Starts a trace at (xs, ys) (capturezone.py:211-219).  Returns true if the
-// integration loop has steps to take.
-template <bool kConfined>
-__device__ __forceinline__ bool dp5_start(const Field64 &f, const Integ &I, Trace64 &s, double xs,
-                                          double ys)
+// Opens a trace at (xs, ys) (capturezone.py:211-217).
+__device__ __forceinline__ void open64(Trace64 &s, const Integ &I, double xs, double ys)
 {
     s.x = xs;
     s.y = ys;
@@ -245,11 +331,51 @@ __device__ __forceinline__ bool dp5_start(const Field64 &f, const Integ &I, Trac
     s.bx0 = s.bx1 = xs;
     s.by0 = s.by1 = ys;
     s.status = OKA_TRACE_OK;
-    if (!feval<kConfined>(f, xs, ys, s.k1x, s.k1y)) {
+}
+
+// Starts an opened trace: k1 = f(start) (capturezone.py:218-219).  Returns
+// true if the integration loop has steps to take.
+template <bool kConfined>
+__device__ __forceinline__ bool dp5_start(const Field64 &f, const Integ &I, Trace64 &s)
+{
+    if (!eval64<kConfined>(f, s.x, s.y, s.k1x, s.k1y)) {
         s.status = OKA_TRACE_TRUNCATED;
         return false;
     }
     return 0.0 < I.absdur;
+}
+
+// The stages of an attempted step.
+struct Stages64 {
+    double k3x, k3y, k4x, k4y, k5x, k5y, k6x, k6y, k7x, k7y, xn, yn;
+};
+
+// Stages 3 to 7 of an attempted step of size dt given k2
+// (capturezone.py:228-240); false where an evaluation raises.
+template <bool kConfined, bool kPlain>
+__device__ __forceinline__ bool dp5_stages(const Field64 &f, const Trace64 &s, double dt,
+                                           double k2x, double k2y, Stages64 &k, bool &ok)
+{
+    const double x = s.x, y = s.y, k1x = s.k1x, k1y = s.k1y;
+    if (!feval<kConfined, kPlain>(f, x + dt * (A31 * k1x + A32 * k2x),
+                                  y + dt * (A31 * k1y + A32 * k2y), k.k3x, k.k3y, ok))
+        return false;
+    if (!feval<kConfined, kPlain>(f, x + dt * ((A41 * k1x + A42 * k2x) + A43 * k.k3x),
+                                  y + dt * ((A41 * k1y + A42 * k2y) + A43 * k.k3y), k.k4x, k.k4y,
+                                  ok))
+        return false;
+    if (!feval<kConfined, kPlain>(
+            f, x + dt * (((A51 * k1x + A52 * k2x) + A53 * k.k3x) + A54 * k.k4x),
+            y + dt * (((A51 * k1y + A52 * k2y) + A53 * k.k3y) + A54 * k.k4y), k.k5x, k.k5y, ok))
+        return false;
+    if (!feval<kConfined, kPlain>(
+            f, x + dt * ((((A61 * k1x + A62 * k2x) + A63 * k.k3x) + A64 * k.k4x) + A65 * k.k5x),
+            y + dt * ((((A61 * k1y + A62 * k2y) + A63 * k.k3y) + A64 * k.k4y) + A65 * k.k5y),
+            k.k6x, k.k6y, ok))
+        return false;
+    k.xn = x + dt * ((((B1 * k1x + B3 * k.k3x) + B4 * k.k4x) + B5 * k.k5x) + B6 * k.k6x);
+    k.yn = y + dt * ((((B1 * k1y + B3 * k.k3y) + B4 * k.k4y) + B5 * k.k5y) + B6 * k.k6y);
+    return feval<kConfined, kPlain>(f, k.xn, k.yn, k.k7x, k.k7y, ok);
 }
 
 // One attempted step of capturezone.py:221-247.  Returns bit 0 = accepted
@@ -263,75 +389,64 @@ __device__ __forceinline__ int dp5_attempt(const Field64 &f, const Integ &I, Tra
         dt = I.dur - s.t;
     s.att += 1;
     const double x = s.x, y = s.y, k1x = s.k1x, k1y = s.k1y;
-    double k2x, k2y, k3x, k3y, k4x, k4y, k5x, k5y, k6x, k6y, k7x, k7y;
-    if (!feval<kConfined>(f, x + dt * (A21 * k1x), y + dt * (A21 * k1y), k2x, k2y))
-        goto trunc;
-    if (!feval<kConfined>(f, x + dt * (A31 * k1x + A32 * k2x), y + dt * (A31 * k1y + A32 * k2y),
-                          k3x, k3y))
-        goto trunc;
-    if (!feval<kConfined>(f, x + dt * ((A41 * k1x + A42 * k2x) + A43 * k3x),
-                          y + dt * ((A41 * k1y + A42 * k2y) + A43 * k3y), k4x, k4y))
-        goto trunc;
-    if (!feval<kConfined>(f, x + dt * (((A51 * k1x + A52 * k2x) + A53 * k3x) + A54 * k4x),
-                          y + dt * (((A51 * k1y + A52 * k2y) + A53 * k3y) + A54 * k4y), k5x, k5y))
-        goto trunc;
-    if (!feval<kConfined>(
-            f, x + dt * ((((A61 * k1x + A62 * k2x) + A63 * k3x) + A64 * k4x) + A65 * k5x),
-            y + dt * ((((A61 * k1y + A62 * k2y) + A63 * k3y) + A64 * k4y) + A65 * k5y), k6x, k6y))
-        goto trunc;
-    {
-        const double xn = x + dt * ((((B1 * k1x + B3 * k3x) + B4 * k4x) + B5 * k5x) + B6 * k6x);
-        const double yn = y + dt * ((((B1 * k1y + B3 * k3y) + B4 * k4y) + B5 * k5y) + B6 * k6y);
-        if (!feval<kConfined>(f, xn, yn, k7x, k7y))
-            goto trunc;
-        const double ex =
-            dt * (((((E1 * k1x + E2 * k7x) + E3 * k3x) + E4 * k4x) + E5 * k5x) + E6 * k6x);
-        const double ey =
-            dt * (((((E1 * k1y + E2 * k7y) + E3 * k3y) + E4 * k4y) + E5 * k5y) + E6 * k6y);
-        const double ax = fabs(ex), ay = fabs(ey);
-        const double est = (isnan(ax) || isnan(ay)) ? (double)NAN : (ay > ax ? ay : ax);
-        const double d0 = xn - x, d1 = yn - y;
-        const double ds = sqrt(fma_(d1, d1, d0 * d0));  // numpy norm: sqrt of a contracted ddot
-        int res = 0;
-        if (est < I.tol && ds < I.maxstep) {
-            s.t = s.t + dt;
-            s.k1x = k7x;
-            s.k1y = k7y;
-            ox = x;
-            oy = y;
-            s.x = xn;
-            s.y = yn;
-            s.acc += 1;
-            s.bx0 = xn < s.bx0 ? xn : s.bx0;
-            s.bx1 = xn > s.bx1 ? xn : s.bx1;
-            s.by0 = yn < s.by0 ? yn : s.by0;
-            s.by1 = yn > s.by1 ? yn : s.by1;
-            res = 1;
-        }
-        double c = pow_fifth(I.tol / (est + kEps));
-        const double c2 = I.maxstep / (ds + kEps);
-        if (c2 < c)
-            c = c2;
-        if (10.0 < c)
-            c = 10.0;
-        dt = (0.9 * c) * dt;
-        s.dt = dt;
-        if (fabs(s.t) < I.absdur) {
-            if (isnan(dt) || dt == 0.0) {
-                s.status = OKA_TRACE_STALLED;
-                res |= 2;
-            } else if (I.cap > 0 && s.att >= I.cap) {
-                s.status = OKA_TRACE_STEP_CAP;
-                res |= 2;
-            }
-        } else {
+    double k2x, k2y;
+    Stages64 k;
+    bool ok = f.plain != kPlainNever;
+    bool wet = eval64<kConfined>(f, x + dt * (A21 * k1x), y + dt * (A21 * k1y), k2x, k2y);
+    if (wet) {
+        if (ok)
+            wet = dp5_stages<kConfined, true>(f, s, dt, k2x, k2y, k, ok);
+        if (__ballot(!ok) != 0ull)
+            wet = dp5_stages<kConfined, false>(f, s, dt, k2x, k2y, k, ok);
+    }
+    if (!wet) {
+        s.status = OKA_TRACE_TRUNCATED;
+        return 2;
+    }
+    const double ex =
+        dt * (((((E1 * k1x + E2 * k.k7x) + E3 * k.k3x) + E4 * k.k4x) + E5 * k.k5x) + E6 * k.k6x);
+    const double ey =
+        dt * (((((E1 * k1y + E2 * k.k7y) + E3 * k.k3y) + E4 * k.k4y) + E5 * k.k5y) + E6 * k.k6y);
+    const double ax = fabs(ex), ay = fabs(ey);
+    const double est = (isnan(ax) || isnan(ay)) ? (double)NAN : (ay > ax ? ay : ax);
+    const double d0 = k.xn - x, d1 = k.yn - y;
+    const double ds = sqrt(fma_(d1, d1, d0 * d0));  // numpy norm: sqrt of a contracted ddot
+    int res = 0;
+    if (est < I.tol && ds < I.maxstep) {
+        s.t = s.t + dt;
+        s.k1x = k.k7x;
+        s.k1y = k.k7y;
+        ox = x;
+        oy = y;
+        s.x = k.xn;
+        s.y = k.yn;
+        s.acc += 1;
+        s.bx0 = k.xn < s.bx0 ? k.xn : s.bx0;
+        s.bx1 = k.xn > s.bx1 ? k.xn : s.bx1;
+        s.by0 = k.yn < s.by0 ? k.yn : s.by0;
+        s.by1 = k.yn > s.by1 ? k.yn : s.by1;
+        res = 1;
+    }
+    double c = pow_fifth(I.tol / (est + kEps));
+    const double c2 = I.maxstep / (ds + kEps);
+    if (c2 < c)
+        c = c2;
+    if (10.0 < c)
+        c = 10.0;
+    dt = (0.9 * c) * dt;
+    s.dt = dt;
+    if (fabs(s.t) < I.absdur) {
+        if (isnan(dt) || dt == 0.0) {
+            s.status = OKA_TRACE_STALLED;
+            res |= 2;
+        } else if (I.cap > 0 && s.att >= I.cap) {
+            s.status = OKA_TRACE_STEP_CAP;
             res |= 2;
         }
-        return res;
+    } else {
+        res |= 2;
     }
-trunc:
-    s.status = OKA_TRACE_TRUNCATED;
-    return 2;
+    return res;
 }
 
 struct EpochReg {

@@ -21,11 +21,11 @@ using namespace pool;
 struct PoolFP64 {
     using Well = Well64;
     struct Consts {
-        double xo, yo, A, B, C, D, E, F, A2, B2, K, bt, bn, por, half_kb2;   // Field64
+        double xo, yo, A, B, C, D, E, F, A2, B2, K, bt, bn, rbn, por, half_kb2;   // Field64
         double dur, absdur, tol, maxstep, sg;                               // Integ
         double gdx, gdy, umbra, u2;
         long long cap;
-        int plain, pad;
+        int plain, pad[3];
     };
     struct Lane {
         Trace64 s;
@@ -37,11 +37,11 @@ struct PoolFP64 {
     };
     static constexpr int kWavesPerEU = 2;
 
-    // Realization r's wells (x, y, -q); returns whether they all allow the
-    // short division sequence (plain_coord, plain_strength).
-    __device__ static bool stage_wells(Well64 *w, const TraceArgs &A, int64_t r)
+    // Realization r's wells (x, y, -q); returns when they allow the short
+    // division sequences (kPlain*).
+    __device__ static int stage_wells(Well64 *w, const TraceArgs &A, int64_t r)
     {
-        int ok = 1;
+        int ok = min(plain_origin(A.xo), plain_origin(A.yo));
         for (int i = threadIdx.x; i < A.nwells; i += kWave) {
             Well64 wl;
             wl.x = A.wells_xy[2 * i];
@@ -49,14 +49,16 @@ struct PoolFP64 {
             wl.nq = -A.q[r * A.nwells + i];
             wl.pad = 0.0;
             w[i] = wl;
-            ok &= plain_coord(wl.x) && plain_coord(wl.y) && plain_strength(wl.nq);
+            ok = min(ok, plain_well(wl));
         }
-        return __ballot(!ok) == 0ull;
+        return __ballot(ok < kPlainBelow) == 0ull   ? kPlainBelow
+               : __ballot(ok < kPlainCoord) == 0ull ? kPlainCoord
+                                                    : kPlainNever;
     }
 
     // make_field and make_integ of the workgroup tracer, per slot.
     __device__ static void stage_consts(Consts &k, const PoolArgs &, const TraceArgs &A, int64_t r,
-                                        int, bool plain)
+                                        int, int plain)
     {
         const double *c = A.coef + 6 * r;
         k.xo = A.xo;
@@ -85,7 +87,8 @@ struct PoolFP64 {
         k.gdy = A.gdy;
         k.umbra = A.umbra;
         k.u2 = A.umbra * A.umbra;
-        k.plain = plain ? 1 : 0;
+        k.rbn = recip_plain(k.bn);
+        k.plain = plain_field(field(k, nullptr, 0)) ? plain : kPlainNever;
     }
 
     __device__ static bool stage_slot(const Consts &, const Well64 *, int) { return false; }
@@ -97,7 +100,7 @@ struct PoolFP64 {
         Field64 f;
         f.w = w;
         f.nw = nw;
-        f.plain = k.plain != 0;
+        f.plain = k.plain;
         f.xo = k.xo;
         f.yo = k.yo;
         f.A = k.A;
@@ -111,6 +114,7 @@ struct PoolFP64 {
         f.K = k.K;
         f.bt = k.bt;
         f.bn = k.bn;
+        f.rbn = k.rbn;
         f.por = k.por;
         f.half_kb2 = k.half_kb2;
         return f;
@@ -151,7 +155,8 @@ struct PoolFP64 {
         const Integ I = integ(k);
         if (ln.fresh) {
             ln.fresh = false;
-            return dp5_start<kConfined>(f, I, ln.s, ln.xs, ln.ys) ? 0 : 2;
+            open64(ln.s, I, ln.xs, ln.ys);
+            return dp5_start<kConfined>(f, I, ln.s) ? 0 : 2;
         }
         double ox, oy;
         const int res = dp5_attempt<kConfined>(f, I, ln.s, ox, oy);

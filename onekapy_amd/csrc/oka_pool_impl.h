@@ -339,7 +339,7 @@ __device__ void open_slot(const PoolArgs &P, const PoolLds<Prec> &L, int s, int6
     const int64_t r = nch > 0 ? local / nch : 0;
     const int ch = nch > 0 ? (int)(local - r * nch) : 0;
     typename Prec::Well *w = L.wells + (size_t)s * P.max_nwells;
-    const bool flag = Prec::stage_wells(w, A, r);
+    const auto flag = Prec::stage_wells(w, A, r);
     if (threadIdx.x == 0) {
         SlotHdr<Prec> &h = L.hdr[s];
         Prec::stage_consts(h.k, P, A, r, s, flag);

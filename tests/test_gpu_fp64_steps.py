@@ -1,0 +1,52 @@
+"""The FP64-exact tracers' rules for their short sequences: each case sits on
+one side of a rule, and the vertices (or counts) must be the oracle's bit for
+bit on either."""
+import numpy as np
+import pytest
+
+import oracle as O
+from onekapy_amd import Realizations, _lib, chronicle_into_field, trace_vertices
+from onekapy_amd.sites import fixed_field
+
+pytestmark = pytest.mark.gpu
+
+COEF = (1e-5, -2e-5, 0.0, 1e-2, -5e-3, 2000.0)
+# wells (x, y, r, q), start point, coefficients A..F, porosity, thickness
+RULES = {
+    # no zero coordinate: only the points' upper bound is checked
+    "all_nonzero": ([(500.0, 300.0, 0.25, 700.0), (900.0, 650.0, 0.25, 400.0)],
+                    (501.25, 300.0), COEF, 0.25, 20.0),
+    # a well and the origin on the axes: points pass the lower bound too,
+    # the first one with a coordinate of exactly 0
+    "zero_well_coordinate": ([(0.0, 0.0, 0.25, 700.0), (0.0, 650.0, 0.25, 400.0)],
+                             (0.0, -1.25), COEF, 0.25, 20.0),
+    "subnormal_start": ([(0.0, 0.0, 0.25, 700.0), (300.0, 650.0, 0.25, 400.0)],
+                        (1.0e-310, 1.25), COEF, 0.25, 20.0),
+    # a regional coefficient below 2^-200, and one above 2^100
+    "tiny_coefficient": ([(500.0, 300.0, 0.25, 700.0)], (501.25, 300.0),
+                         (1e-5, -2e-5, 1e-70, 1e-2, -5e-3, 2000.0), 0.25, 20.0),
+    "huge_coefficient": ([(500.0, 300.0, 0.25, 700.0)], (501.25, 300.0),
+                         (1e-5, -2e-5, 0.0, 2e30, -5e-3, 2000.0), 0.25, 20.0),
+    # thickness x porosity below 2^-100
+    "tiny_bn": ([(500.0, 300.0, 0.25, 7e-29)], (501.25, 300.0),
+                (1e-38, -2e-38, 0.0, 1e-35, -5e-36, 2000.0), 1e-16, 1e-16),
+    # stages far beyond 2^60: a start within rounding of a well
+    "stage_overflow": ([(500.0, 300.0, 0.25, 1e30), (900.0, 650.0, 0.25, 400.0)],
+                       (500.0 + 2.0 ** -40, 300.0), COEF, 0.25, 20.0),
+}
+
+
+@pytest.mark.parametrize("case", sorted(RULES))
+def test_short_division_rules_bit_exact_vs_oracle(gpu_ctx, case):
+    wells, start, coef, por, thick = RULES[case]
+    w = np.array(wells, dtype=float)
+    xo, yo = w[0, 0], w[0, 1]
+    real = Realizations([10.0], [por], [thick], w[:, 3].reshape(1, -1), np.array(coef, float))
+    om = O.OracleModel(0.0, 10.0, por, thick, w, xo, yo, coef)
+    cap = 400
+    verts, nverts, status = trace_vertices(np.ascontiguousarray(w[:, :2]), xo, yo, real,
+                                           np.array([start]), 300.0, 1.0, 10.0, True, cap)
+    ov, res = om.backtrace(start[0], start[1], 300.0, 1.0, 10.0, confined=True, max_steps=cap)
+    assert (status[0], nverts[0]) == (res.status, res.nverts)
+    assert np.array_equal(verts[0, :nverts[0]], ov)
+    assert np.array_equal(np.signbit(verts[0, :nverts[0]]), np.signbit(ov))

@@ -141,7 +141,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
         EpochReg ep;
         int p = tid;
         bool have = p < P;
-        bool live = false;
+        bool live = false, fresh = false;
         for (;;) {
             bool ended = false;
             int64_t k = (int64_t)r * P + p;
@@ -156,24 +156,22 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
                     a.verts[2 * (k * a.vcap) + 1] = ys;
                 }
                 open64(s, I, xs, ys);
-                live = dp5_start<kConfined>(f, I, s);
-                ended = !live;
-            } else {
-                double ox, oy;
-                const int res = dp5_attempt<kConfined>(f, I, s, ox, oy);
-                if (res & 1) {
-                    if (raster)
-                        n_cand += (unsigned long long)raster_segment(ch.bits, ep, a.gdx, a.gdy,
-                                                                     umbra, u2, ox, oy, s.x, s.y);
-                    if (kVerts && s.acc < a.vcap) {
-                        a.verts[2 * (k * a.vcap + s.acc)] = s.x;
-                        a.verts[2 * (k * a.vcap + s.acc) + 1] = s.y;
-                    }
+                live = fresh = true;
+            }
+            double ox, oy;
+            const int res = advance64<kConfined>(f, I, s, fresh, ox, oy);
+            if (res & 1) {
+                if (raster)
+                    n_cand += (unsigned long long)raster_segment(ch.bits, ep, a.gdx, a.gdy, umbra,
+                                                                 u2, ox, oy, s.x, s.y);
+                if (kVerts && s.acc < a.vcap) {
+                    a.verts[2 * (k * a.vcap + s.acc)] = s.x;
+                    a.verts[2 * (k * a.vcap + s.acc) + 1] = s.y;
                 }
-                if (res & 2) {
-                    live = false;
-                    ended = true;
-                }
+            }
+            if (res & 2) {
+                live = false;
+                ended = true;
             }
             if (ended) {
                 n_att += (unsigned long long)s.att;

@@ -319,30 +319,20 @@ struct Trace64 {
     int status;
 };
 
-// Opens a trace at (xs, ys) (capturezone.py:211-217).
+// Opens a trace at (xs, ys) (capturezone.py:211-217).  Its k1 = f(start) is
+// the next advance64's evaluation.
 __device__ __forceinline__ void open64(Trace64 &s, const Integ &I, double xs, double ys)
 {
     s.x = xs;
     s.y = ys;
     s.t = 0.0;
     s.dt = 0.1 * I.sg;
+    s.k1x = s.k1y = 0.0;
     s.att = 0;
     s.acc = 0;
     s.bx0 = s.bx1 = xs;
     s.by0 = s.by1 = ys;
     s.status = OKA_TRACE_OK;
-}
-
-// Starts an opened trace: k1 = f(start) (capturezone.py:218-219).  Returns
-// true if the integration loop has steps to take.
-template <bool kConfined>
-__device__ __forceinline__ bool dp5_start(const Field64 &f, const Integ &I, Trace64 &s)
-{
-    if (!eval64<kConfined>(f, s.x, s.y, s.k1x, s.k1y)) {
-        s.status = OKA_TRACE_TRUNCATED;
-        return false;
-    }
-    return 0.0 < I.absdur;
 }
 
 // The stages of an attempted step.
@@ -378,21 +368,34 @@ __device__ __forceinline__ bool dp5_stages(const Field64 &f, const Trace64 &s, d
     return feval<kConfined, kPlain>(f, k.xn, k.yn, k.k7x, k.k7y, ok);
 }
 
-// One attempted step of capturezone.py:221-247.  Returns bit 0 = accepted
-// (segment (ox, oy) -> (s.x, s.y)), bit 1 = the trace has ended.
+// One iteration of a trace: k1 of a fresh trace (capturezone.py:218-219), else
+// an attempted step (capturezone.py:221-247).  Returns bit 0 = accepted
+// (segment (ox, oy) -> (s.x, s.y)), bit 1 = the trace has ended.  A fresh
+// trace's k1 is its lane's share of the evaluation that the wave's other
+// lanes spend on their step's second stage, so starting a trace costs the
+// wave no evaluation of its own.
 template <bool kConfined>
-__device__ __forceinline__ int dp5_attempt(const Field64 &f, const Integ &I, Trace64 &s,
-                                           double &ox, double &oy)
+__device__ __forceinline__ int advance64(const Field64 &f, const Integ &I, Trace64 &s, bool &fresh,
+                                         double &ox, double &oy)
 {
     double dt = s.dt;
     if (fabs(s.t + dt) > I.absdur)
         dt = I.dur - s.t;
-    s.att += 1;
     const double x = s.x, y = s.y, k1x = s.k1x, k1y = s.k1y;
     double k2x, k2y;
+    bool wet = eval64<kConfined>(f, fresh ? x : x + dt * (A21 * k1x),
+                                 fresh ? y : y + dt * (A21 * k1y), k2x, k2y);
+    if (fresh) {
+        fresh = false;
+        s.k1x = k2x;
+        s.k1y = k2y;
+        if (!wet)
+            s.status = OKA_TRACE_TRUNCATED;
+        return wet && 0.0 < I.absdur ? 0 : 2;
+    }
+    s.att += 1;
     Stages64 k;
     bool ok = f.plain != kPlainNever;
-    bool wet = eval64<kConfined>(f, x + dt * (A21 * k1x), y + dt * (A21 * k1y), k2x, k2y);
     if (wet) {
         if (ok)
             wet = dp5_stages<kConfined, true>(f, s, dt, k2x, k2y, k, ok);

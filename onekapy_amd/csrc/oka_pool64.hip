@@ -30,10 +30,9 @@ struct PoolFP64 {
     struct Lane {
         Trace64 s;
         EpochReg ep;
-        double xs, ys;             // start point of a fresh trace
         unsigned long long cand;   // candidate nodes of the trace
         uint32_t last_t, last_v;   // the lane's tile cache (PoolBits::lookup)
-        bool fresh;                // not yet started (k1 not evaluated)
+        bool fresh;                // k1 not yet evaluated
     };
     static constexpr int kWavesPerEU = 2;
 
@@ -132,34 +131,28 @@ struct PoolFP64 {
         return I;
     }
 
-    __device__ static void open(Lane &ln, const Consts &, const TraceArgs &A, int64_t r, int p,
+    __device__ static void open(Lane &ln, const Consts &k, const TraceArgs &A, int64_t r, int p,
                                 bool raster)
     {
         if (raster)
             ln.ep = find_epoch(A, r * A.npaths + p);
-        ln.xs = A.start_xy[2 * p];
-        ln.ys = A.start_xy[2 * p + 1];
+        open64(ln.s, integ(k), A.start_xy[2 * p], A.start_xy[2 * p + 1]);
         ln.cand = 0;
         ln.last_t = kKeyEmpty;
         ln.last_v = kValNone;
         ln.fresh = true;
     }
 
-    // A fresh trace evaluates k1 at its start (capturezone.py:211-219); every
-    // other iteration is one attempted step (capturezone.py:221-247).
+    // One field evaluation for every lane (k1 of a fresh trace, else the step's
+    // second stage), then the rest of the attempted steps.
     template <bool kConfined>
     __device__ static int advance(Lane &ln, const Consts &k, const Well64 *w, int nw,
                                   PoolBits &bits, bool raster)
     {
         const Field64 f = field(k, w, nw);
         const Integ I = integ(k);
-        if (ln.fresh) {
-            ln.fresh = false;
-            open64(ln.s, I, ln.xs, ln.ys);
-            return dp5_start<kConfined>(f, I, ln.s) ? 0 : 2;
-        }
         double ox, oy;
-        const int res = dp5_attempt<kConfined>(f, I, ln.s, ox, oy);
+        const int res = advance64<kConfined>(f, I, ln.s, ln.fresh, ox, oy);
         if ((res & 1) && raster) {
             bits.last_t = ln.last_t;
             bits.last_v = ln.last_v;

@@ -675,7 +675,8 @@ int oka_fit_draw(oka_ctx *c, const oka_site *site, int32_t nreal, const double *
     TRY(stage_in(c, kSlotZ, z, sizeof(double) * 6 * nreal, flags, &d));
     a.z = (const double *)d;
     void *o;
-    TRY(ensure(c, kSlotLogs, sizeof(double) * site->nobs * std::max(site->nwells, 1), &o));
+    TRY(ensure(c, kSlotLogs, sizeof(double) * fit_logs_count(site->nobs, std::max(site->nwells, 1)),
+               &o));
     a.logr2 = (const double *)o;
     TRY(stage_out(c, kSlotEv, ev, sizeof(double) * 6 * nreal, flags, false, &o));
     a.ev = (double *)o;

@@ -24,7 +24,8 @@ struct oka_batch {
     PoolShape shape;
     void *d_sites = nullptr, *d_first = nullptr, *d_queue = nullptr;
     void *d_fits = nullptr, *d_fit_first = nullptr;   // fit table, its two prefix arrays
-    int64_t fit_logs = 0, fit_reals = 0;
+    int64_t fit_logs = 0, fit_groups = 0;
+    int max_nobs = 0;
     void *d_hbm = nullptr, *d_rec = nullptr, *d_beta = nullptr;
     size_t hbm_cap = 0, rec_cap = 0, first_cap = 0, beta_cap = 0;
     hipGraphExec_t exec = nullptr;
@@ -99,7 +100,7 @@ int stage_site(oka_batch *B, int s, const oka_batch_site &bs)
     TRY(bcopy(B, bs.z, (size_t)6 * nr, &f.z));
     TRY(bcopy(B, o.start_xy, (size_t)2 * o.npaths, &a.start_xy));
     void *p;
-    TRY(balloc(B, sizeof(double) * site->nobs * std::max(nw, 1), &p));
+    TRY(balloc(B, sizeof(double) * fit_logs_count(site->nobs, std::max(nw, 1)), &p));
     f.logr2 = (const double *)p;
     TRY(balloc(B, sizeof(double) * 6 * std::max(nr, 1), &p));
     f.coef = (double *)p;
@@ -194,7 +195,7 @@ int capture(oka_batch *B)
         (launch_fit_logs_multi((const FitArgs *)B->d_fits, B->nsites, ff, B->fit_logs,
                                c->stream) != hipSuccess ||
          launch_fit_draw_multi((const FitArgs *)B->d_fits, B->nsites, ff + B->nsites + 1,
-                               B->fit_reals, c->stream) != hipSuccess))
+                               B->fit_groups, B->max_nobs, c->stream) != hipSuccess))
         rc = fail(c, OKA_ERR_DEVICE, "fit launch failed");
     if (rc == OKA_OK)
         rc = pool_launch(c, sh, p);
@@ -242,16 +243,16 @@ int oka_batch_create(oka_ctx *c, int32_t nsites, const oka_batch_site *sites,
         rc = fail(c, OKA_ERR_DEVICE, "batch staging failed");
     rc = rc ? rc : balloc(B, sizeof(unsigned long long), &B->d_queue);
     if (rc == OKA_OK) {
-        // fit table and the prefix sums of its (observation, well) pairs and realizations
+        // fit table and the prefix sums of its logarithms and workgroups
         std::vector<int64_t> ff(2 * ((size_t)nsites + 1), 0);
         for (int s = 0; s < nsites; ++s) {
             const FitArgs &f = B->fits[s];
-            const int64_t logs = f.nreal > 0 ? (int64_t)f.nobs * f.nwells : 0;
-            ff[s + 1] = ff[s] + logs;
-            ff[nsites + 1 + s + 1] = ff[nsites + 1 + s] + f.nreal;
+            ff[s + 1] = ff[s] + (f.nreal > 0 ? fit_logs_count(f.nobs, f.nwells) : 0);
+            ff[nsites + 1 + s + 1] = ff[nsites + 1 + s] + fit_blocks(f.nreal);
+            B->max_nobs = std::max(B->max_nobs, f.nreal > 0 ? (int)f.nobs : 0);
         }
         B->fit_logs = ff[nsites];
-        B->fit_reals = ff[2 * (size_t)nsites + 1];
+        B->fit_groups = ff[2 * (size_t)nsites + 1];
         rc = balloc(B, sizeof(FitArgs) * nsites, &B->d_fits);
         rc = rc ? rc : balloc(B, sizeof(int64_t) * ff.size(), &B->d_fit_first);
         if (rc == OKA_OK &&

@@ -373,7 +373,7 @@ struct FitArgs {
     const double *wells_xy;     // nwells x 2
     const double *obs;          // nobs x 4
     double xo, yo, base;
-    const double *logr2;        // nobs x nwells: log(r^2) observation to well
+    const double *logr2;        // nwells x fit_obs_stride(nobs): log(r^2) well to observation
     const double *K, *b, *q, *z;
     double *ev, *cov, *coef;
     int32_t *status;
@@ -488,13 +488,21 @@ hipError_t launch_trace_fp32(const TraceArgs &a, int grid_blocks, int kind,
 size_t trace_fp32_wells_lds(int nwells);
 
 // oka_fit.hip
+// Doubles between two wells' logarithms (64-byte rows) and of all of them.
+__host__ __device__ inline int fit_obs_stride(int nobs) { return (nobs + 7) / 8 * 8; }
+__host__ __device__ inline int64_t fit_logs_count(int nobs, int nwells)
+{
+    return (int64_t)fit_obs_stride(nobs) * nwells;
+}
+int64_t fit_blocks(int64_t nreal);   // workgroups of one site's fit and draw
 hipError_t launch_fit_logs(const FitArgs &a, double *logr2, hipStream_t s);
-// Over a device table of sites; `first` holds the prefix sums of the item
-// counts (nobs x nwells for the logs, nreal for the fits), total the last.
+// Over a device table of sites; `first` holds the prefix sums of
+// fit_logs_count for the logs and of fit_blocks for the fits, total or blocks
+// their last, max_nobs the most observations of a site.
 hipError_t launch_fit_logs_multi(const FitArgs *sites, int nsites, const int64_t *first,
                                  int64_t total, hipStream_t s);
 hipError_t launch_fit_draw_multi(const FitArgs *sites, int nsites, const int64_t *first,
-                                 int64_t total, hipStream_t s);
+                                 int64_t blocks, int max_nobs, hipStream_t s);
 hipError_t launch_fit_draw(const FitArgs &a, hipStream_t s);
 
 double host_pow_fifth(double x);

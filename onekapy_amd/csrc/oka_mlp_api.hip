@@ -838,11 +838,12 @@ static int cv_sums(oka_ctx *c, oka_mlp *M, const oka_site *site, const oka_dist 
     const int64_t total = batched ? n * nrep : n;
     const int32_t runs = batched ? 1 : nrep;
     // site, distributions, standardization (host memory)
-    const size_t site_doubles = (size_t)2 * nw + 4 * nobs + (size_t)nobs * nw + 2 * nin;
+    const size_t n_logs = (size_t)fit_logs_count(nobs, nw);
+    const size_t site_doubles = n_logs + (size_t)2 * nw + 4 * nobs + 2 * nin;
     void *sb;
     TRY(ensure(c, kSlotCvSite, sizeof(double) * site_doubles, &sb));
-    double *d_wells = (double *)sb, *d_obs = d_wells + 2 * nw, *d_logr2 = d_obs + 4 * nobs;
-    double *d_mean = d_logr2 + (size_t)nobs * nw, *d_std = d_mean + nin;
+    double *d_logr2 = (double *)sb, *d_wells = d_logr2 + n_logs, *d_obs = d_wells + 2 * nw;
+    double *d_mean = d_obs + 4 * nobs, *d_std = d_mean + nin;
     HIPCHK(c, hipMemcpyAsync(d_wells, site->wells_xy, sizeof(double) * 2 * nw,
                              hipMemcpyHostToDevice, s));
     HIPCHK(c, hipMemcpyAsync(d_obs, site->obs, sizeof(double) * 4 * nobs, hipMemcpyHostToDevice, s));

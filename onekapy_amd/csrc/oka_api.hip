@@ -476,6 +476,10 @@ int check_opts(oka_ctx *c, const oka_trace_opts *o)
 
 constexpr int64_t kDefaultMaxSteps = 1000000;
 
+// The workgroup schedule takes as many wells as whole records of them (32
+// bytes in FP64, 16 in FP32) fit in a workgroup's LDS.
+size_t wells_limit_lds(int nwells, bool fp64) { return (size_t)nwells * (fp64 ? 32 : 16); }
+
 }  // namespace
 
 extern "C" {
@@ -1059,7 +1063,7 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
     // launch shape: one realization per 256-lane workgroup, grid-stride
     const size_t base_lds =
         (fp64 ? trace_fp64_wells_lds(a.nwells) : trace_fp32_wells_lds(a.nwells)) + win_lds;
-    if (base_lds > c->max_lds)
+    if (wells_limit_lds(a.nwells, fp64) + win_lds > c->max_lds)
         return fail(c, OKA_ERR_ARG, "too many wells for LDS (%d)", a.nwells);
     int kind = kBmLdsFlat;
     int blocks = nreal;
@@ -1206,7 +1210,7 @@ int oka_trace_chronicle_noalloc(oka_ctx *c, const oka_site *site, int32_t nreal,
 
     const bool fp64 = o->precision == OKA_FP64_EXACT;
     const size_t base_lds = fp64 ? trace_fp64_wells_lds(a.nwells) : trace_fp32_wells_lds(a.nwells);
-    if (base_lds > c->max_lds)
+    if (wells_limit_lds(a.nwells, fp64) > c->max_lds)
         return fail(c, OKA_ERR_ARG, "too many wells for LDS (%d)", a.nwells);
     int kind = kBmLdsFlat;
     int blocks = nreal;

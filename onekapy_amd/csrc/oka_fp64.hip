@@ -11,7 +11,7 @@
 //
 // Work layout: one workgroup per realization (grid-stride over realizations),
 // one particle per lane with lanes refilled from an LDS counter as their traces
-// end, the realization's wells staged in LDS, and the realization's visited-node
+// end, the realization's discharges staged in LDS, and the realization's visited-node
 // bitmap in LDS (or HBM for grids too large for it).  At the end of the
 // realization the bitmap is flushed into the int32 count grid with one atomic
 // add per set bit, so a node counts once per realization
@@ -85,7 +85,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
 {
     constexpr bool kVerts = kMode == kModeVertices;
     extern __shared__ double smem[];
-    Well64 *s_wells = reinterpret_cast<Well64 *>(smem);
+    double *s_nq = smem;   // the realization's -q
     __shared__ int s_next;
     __shared__ unsigned long long s_stat[kStatCount];
 
@@ -95,7 +95,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
     const double umbra = a.umbra;
     const double u2 = umbra * umbra;
     const bool raster = !kVerts && a.rasterize;
-    uint32_t *lds_tail = reinterpret_cast<uint32_t *>(s_wells + a.nwells);
+    uint32_t *lds_tail = reinterpret_cast<uint32_t *>(s_nq + a.nwells);
     Chron<kMode> ch;
     if constexpr (kMode == kModeLdsBitmap) {
         ch.bits = FlatBits{lds_tail, a.gncols};
@@ -121,8 +121,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
             wl.x = a.wells_xy[2 * i];
             wl.y = a.wells_xy[2 * i + 1];
             wl.nq = -a.q[(int64_t)r * a.nwells + i];
-            wl.pad = 0.0;
-            s_wells[i] = wl;
+            s_nq[i] = wl.nq;
             ok = min(ok, plain_well(wl));
         }
         if (raster)
@@ -133,7 +132,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
                           : __syncthreads_and(ok >= kPlainCoord) ? kPlainCoord
                                                                  : kPlainNever;
 
-        const Field64 f = make_field(a, r, s_wells, __builtin_amdgcn_readfirstlane(plain));
+        const FieldSite f = make_field(a, r, s_nq, __builtin_amdgcn_readfirstlane(plain));
         unsigned long long n_att = 0, n_acc = 0, n_esc = 0, n_cand = 0;
         unsigned long long n_st[4] = {0, 0, 0, 0};
 
@@ -322,7 +321,7 @@ hipError_t launch_mode(const TraceArgs &a, int grid_blocks, size_t lds, hipStrea
 
 }  // namespace
 
-size_t trace_fp64_wells_lds(int nwells) { return (size_t)nwells * sizeof(Well64); }
+size_t trace_fp64_wells_lds(int nwells) { return (size_t)nwells * sizeof(double); }
 
 hipError_t launch_trace_fp64(const TraceArgs &a, int grid_blocks, int kind, hipStream_t s)
 {

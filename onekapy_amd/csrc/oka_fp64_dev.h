@@ -45,9 +45,8 @@ struct __align__(16) Well64 {
     double x, y, nq, pad;
 };
 
-// One realization's velocity field.  Wells are typically in LDS.
+// One realization's velocity field, but for its wells.
 struct Field64 {
-    const Well64 *w;
     int nw;
     int plain;           // kPlain*: when the short division sequences apply
     double xo, yo;
@@ -56,6 +55,33 @@ struct Field64 {
     double K, bt, bn;    // conductivity, thickness, thickness*porosity
     double rbn;          // recip_plain(bn)
     double por, half_kb2;
+};
+
+// The field with its wells in LDS, a record each (the pool, whose lanes may be
+// on different sites).
+struct FieldLds : Field64 {
+    const Well64 *w;
+    static constexpr int kBlock = 2;   // wells per loop iteration (confined)
+    __device__ __forceinline__ Well64 well(int i) const { return w[i]; }
+};
+
+// The field of a workgroup that is on one site: the wells' places come by
+// scalar loads from the site's array (wave-uniform, in the scalar cache for
+// every realization), and only the strengths are in LDS.  A broadcast LDS read
+// of 16 bytes takes 16 cycles of the CU's LDS, so with whole records the four
+// SIMDs' 24 bytes a well kept the LDS nearly as busy as their 24 issue slots
+// kept them; a lone trace waits for one round trip per 4 wells instead of per
+// 2.  Against records: 100 x 100 particles of a 4-well site 3 % less time,
+// 10^4 x 1000 of a 25-well site 1-2 %.
+typedef const __attribute__((address_space(4))) double *ConstF64;   // constant: scalar loads
+struct FieldSite : Field64 {
+    ConstF64 xy;         // nw x 2
+    const double *nq;    // LDS
+    static constexpr int kBlock = 4;
+    __device__ __forceinline__ Well64 well(int i) const
+    {
+        return {xy[2 * i], xy[2 * i + 1], nq[i], 0.0};
+    }
 };
 
 // a1 / b and a2 / b, each correctly rounded (IEEE division, as numpy's).
@@ -188,11 +214,12 @@ __device__ __forceinline__ bool plain_point(const Field64 &f, double x, double y
                                   : plain_coord(x) && plain_coord(y);
 }
 
-__device__ __forceinline__ Field64 make_field(const TraceArgs &a, int r, const Well64 *w,
-                                              int plain)
+__device__ __forceinline__ FieldSite make_field(const TraceArgs &a, int r, const double *nq,
+                                                int plain)
 {
-    Field64 f;
-    f.w = w;
+    FieldSite f;
+    f.xy = (ConstF64)a.wells_xy;
+    f.nq = nq;
     f.nw = a.nwells;
     f.xo = a.xo;
     f.yo = a.yo;
@@ -217,17 +244,11 @@ __device__ __forceinline__ Field64 make_field(const TraceArgs &a, int r, const W
 
 // The wells' part of the discharge at (x, y) (model.py:307-313) and, for the
 // unconfined field, of the potential (model.py:258-264).
-template <bool kConfined, bool kPlain>
-__device__ __forceinline__ void well_sums(const Field64 &f, double x, double y, double &Qx,
-                                          double &Qy, double &pw)
+template <bool kConfined, bool kPlain, class F>
+__device__ __forceinline__ void well_sums(const F &f, double x, double y, double &Qx, double &Qy,
+                                          double &pw)
 {
-    // two wells per iteration in the confined field: one LDS address and
-    // loop step serve both (2 % on the 25-well site; by 4 gains nothing, and
-    // the unconfined loop, with its logarithms, is slower unrolled)
-    constexpr int kUnroll = kConfined ? 2 : 1;
-#pragma unroll kUnroll
-    for (int w = 0; w < f.nw; ++w) {
-        const Well64 wl = f.w[w];
+    auto term = [&](const Well64 &wl) {
         const double ddx = x - wl.x;
         const double ddy = y - wl.y;
         const double r2 = ddx * ddx + ddy * ddy;
@@ -243,15 +264,31 @@ __device__ __forceinline__ void well_sums(const Field64 &f, double x, double y, 
         Qy = Qy + sy * kC2Pi;
         if (!kConfined)
             pw = pw + ((-wl.nq) * log_rn(r2)) * kC4Pi;
+    };
+    // several wells per iteration in the confined field, their loads issued
+    // together (the unconfined loop, with its logarithms, is slower unrolled)
+    constexpr int kBlock = kConfined && kPlain ? F::kBlock : 1;
+    int w = 0;
+    for (; w + kBlock <= f.nw; w += kBlock) {
+        Well64 wl[kBlock];
+#pragma unroll
+        for (int k = 0; k < kBlock; ++k)
+            wl[k] = f.well(w + k);
+#pragma unroll
+        for (int k = 0; k < kBlock; ++k)
+            term(wl[k]);
     }
+    if (kBlock > 1)
+        for (; w < f.nw; ++w)
+            term(f.well(w));
 }
 
 // feval(xy) = -V(xy) (stochastic.py:253-260).  Returns false where the
 // reference raises AquiferError (unconfined only).  kPlain uses the short
 // division sequences and clears `ok` when (x, y) does not allow them: the
 // result is then discarded and computed again without kPlain.
-template <bool kConfined, bool kPlain>
-__device__ __forceinline__ bool feval(const Field64 &f, double x, double y, double &kx, double &ky,
+template <bool kConfined, bool kPlain, class F>
+__device__ __forceinline__ bool feval(const F &f, double x, double y, double &kx, double &ky,
                                       bool &ok)
 {
     const double dx = x - f.xo;
@@ -296,8 +333,8 @@ __device__ __forceinline__ bool feval(const Field64 &f, double x, double y, doub
 // again without them when the field or any lane's point does not allow them.
 // Both give the same bits where they apply, so one such lane may take its
 // wave along, and the long sequence stays off the usual path.
-template <bool kConfined>
-__device__ __forceinline__ bool eval64(const Field64 &f, double x, double y, double &kx, double &ky)
+template <bool kConfined, class F>
+__device__ __forceinline__ bool eval64(const F &f, double x, double y, double &kx, double &ky)
 {
     bool ok = f.plain != kPlainNever, wet = false;
     if (ok)
@@ -342,8 +379,8 @@ struct Stages64 {
 
 // Stages 3 to 7 of an attempted step of size dt given k2
 // (capturezone.py:228-240); false where an evaluation raises.
-template <bool kConfined, bool kPlain>
-__device__ __forceinline__ bool dp5_stages(const Field64 &f, const Trace64 &s, double dt,
+template <bool kConfined, bool kPlain, class F>
+__device__ __forceinline__ bool dp5_stages(const F &f, const Trace64 &s, double dt,
                                            double k2x, double k2y, Stages64 &k, bool &ok)
 {
     const double x = s.x, y = s.y, k1x = s.k1x, k1y = s.k1y;
@@ -374,8 +411,8 @@ __device__ __forceinline__ bool dp5_stages(const Field64 &f, const Trace64 &s, d
 // trace's k1 is its lane's share of the evaluation that the wave's other
 // lanes spend on their step's second stage, so starting a trace costs the
 // wave no evaluation of its own.
-template <bool kConfined>
-__device__ __forceinline__ int advance64(const Field64 &f, const Integ &I, Trace64 &s, bool &fresh,
+template <bool kConfined, class F>
+__device__ __forceinline__ int advance64(const F &f, const Integ &I, Trace64 &s, bool &fresh,
                                          double &ox, double &oy)
 {
     double dt = s.dt;

@@ -94,9 +94,9 @@ struct PoolFP64 {
     __device__ static bool table_shared(const Consts &) { return false; }
     __device__ static void table_to(Consts &, float2 *) {}
 
-    __device__ static Field64 field(const Consts &k, const Well64 *w, int nw)
+    __device__ static FieldLds field(const Consts &k, const Well64 *w, int nw)
     {
-        Field64 f;
+        FieldLds f;
         f.w = w;
         f.nw = nw;
         f.plain = k.plain;
@@ -149,7 +149,7 @@ struct PoolFP64 {
     __device__ static int advance(Lane &ln, const Consts &k, const Well64 *w, int nw,
                                   PoolBits &bits, bool raster)
     {
-        const Field64 f = field(k, w, nw);
+        const FieldLds f = field(k, w, nw);
         const Integ I = integ(k);
         double ox, oy;
         const int res = advance64<kConfined>(f, I, ln.s, ln.fresh, ox, oy);

@@ -23,7 +23,9 @@ using namespace oka;
 // process ends.  In host code `scratch` is only a stand-in for the symbol:
 // kernels get the device address that hipGetSymbolAddress returns for the
 // current device (oka_ctx::scratch).
-static __device__ __align__(256) uint32_t scratch[OKA_NOALLOC_SCRATCH_BYTES / 4];
+// Behind its OKA_NOALLOC_SCRATCH_BYTES lie the FP32 tracer's well places.
+constexpr size_t kScrWells = 10240 * sizeof(float2);   // wells_limit_lds allows no more
+static __device__ __align__(256) uint32_t scratch[(OKA_NOALLOC_SCRATCH_BYTES + kScrWells) / 4];
 
 namespace {
 
@@ -1062,7 +1064,8 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
 
     // launch shape: one realization per 256-lane workgroup, grid-stride
     const size_t base_lds =
-        (fp64 ? trace_fp64_wells_lds(a.nwells) : trace_fp32_wells_lds(a.nwells)) + win_lds;
+        (fp64 ? trace_fp64_wells_lds(a.nwells) : trace_fp32_wells_lds(a.nwells, a.confined)) +
+        win_lds;
     if (wells_limit_lds(a.nwells, fp64) + win_lds > c->max_lds)
         return fail(c, OKA_ERR_ARG, "too many wells for LDS (%d)", a.nwells);
     int kind = kBmLdsFlat;
@@ -1083,6 +1086,11 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
             if (kind == kBmTiled)   // overflow tiles start empty; each flush leaves them so
                 TRY(fill_u32(c, a.gbitmap, (int64_t)words * blocks));
         }
+    }
+    if (!fp64) {   // grown in steps of 8,192 wells
+        TRY(ensure(c, kSlotWells32, sizeof(float2) * ((a.nwells + 8191) / 8192 * 8192), &o2));
+        a.wells32 = (const float2 *)o2;
+        HIPCHK(c, launch_site_wells32(a, (float2 *)o2, c->stream));
     }
     if (timed)
         HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -1209,7 +1217,8 @@ int oka_trace_chronicle_noalloc(oka_ctx *c, const oka_site *site, int32_t nreal,
     a.trace_steps = trace_steps;
 
     const bool fp64 = o->precision == OKA_FP64_EXACT;
-    const size_t base_lds = fp64 ? trace_fp64_wells_lds(a.nwells) : trace_fp32_wells_lds(a.nwells);
+    const size_t base_lds = fp64 ? trace_fp64_wells_lds(a.nwells)
+                                 : trace_fp32_wells_lds(a.nwells, a.confined);
     if (wells_limit_lds(a.nwells, fp64) > c->max_lds)
         return fail(c, OKA_ERR_ARG, "too many wells for LDS (%d)", a.nwells);
     int kind = kBmLdsFlat;
@@ -1236,6 +1245,13 @@ int oka_trace_chronicle_noalloc(oka_ctx *c, const oka_site *site, int32_t nreal,
             if (kind == kBmTiled)   // overflow tiles start empty; each flush leaves them so
                 TRY(fill_u32(c, a.gbitmap, per_block * blocks));
         }
+    }
+    if (!fp64) {
+        if (sizeof(float2) * (size_t)a.nwells > kScrWells)
+            return fail(c, OKA_ERR_ARG, "too many wells for LDS (%d)", a.nwells);
+        float2 *w32 = reinterpret_cast<float2 *>(scr + OKA_NOALLOC_SCRATCH_BYTES);
+        a.wells32 = w32;
+        HIPCHK(c, launch_site_wells32(a, w32, c->stream));
     }
     if (stats)
         HIPCHK(c, hipEventRecord(c->ev0, c->stream));

@@ -16,16 +16,18 @@ namespace {
 
 using namespace fp32;
 
-// At most 128 VGPRs, so that 4 waves share a SIMD: the tracer is bound by
-// VALU issue, and with 3 waves (the compiler's own choice, 129 VGPRs) the
-// SIMDs idle about 12 % of the time on LDS and scalar waits.
+// At most 128 VGPRs, so that at least 4 waves share a SIMD: the tracer is
+// bound by VALU issue, and with 3 waves the SIMDs idled about 12 % of the time
+// on LDS and scalar waits.
 template <int kKind, bool kConfined>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4)))
 k_trace_fp32(TraceArgs a)
 {
     extern __shared__ float4 smem4[];
-    float4 *s_w = smem4;
-    uint32_t *s_bm = reinterpret_cast<uint32_t *>(smem4 + a.nwells);
+    // strengths, then (unconfined) the potential's, of 4 wells a float4
+    const int nw4 = (a.nwells + 3) / 4;
+    float *s_q = reinterpret_cast<float *>(smem4), *s_p = reinterpret_cast<float *>(smem4 + nw4);
+    uint32_t *s_bm = reinterpret_cast<uint32_t *>(smem4 + (kConfined ? 1 : 2) * nw4);
     using Bits = typename std::conditional<kKind == kBmTiled, TileBits, FlatBits>::type;
     __shared__ int s_next;
     __shared__ unsigned long long s_stat[kStatCount];
@@ -74,10 +76,9 @@ k_trace_fp32(TraceArgs a)
         const double h = kConfined ? 1.0 : 0.5 * a.K[r] * (a.b[r] * a.b[r]);
         for (int i = tid; i < a.nwells; i += blockDim.x) {
             const double qw = a.q[(int64_t)r * a.nwells + i];
-            s_w[i] = make_float4((float)(a.wells_xy[2 * i] - a.xo),
-                                 (float)(a.wells_xy[2 * i + 1] - a.yo),
-                                 (float)(qw * kInv2Pi / bn),
-                                 kConfined ? 0.0f : (float)(qw * (kInv4Pi * kLn2) / h));
+            s_q[i] = (float)(qw * kInv2Pi / bn);
+            if constexpr (!kConfined)
+                s_p[i] = (float)(qw * (kInv4Pi * kLn2) / h);
         }
         if (tid == 0) {
             const double *c = a.coef + 6 * (int64_t)r;
@@ -97,8 +98,10 @@ k_trace_fp32(TraceArgs a)
         }
         __syncthreads();
 
-        Field32 f;
-        f.w = s_w;
+        Field32Site f;
+        f.xy = (ConstF32)a.wells32;
+        f.q4 = smem4;
+        f.p4 = smem4 + nw4;
         f.nw = a.nwells;
         f.a2 = s_reg[0];
         f.b2 = s_reg[1];
@@ -155,7 +158,8 @@ k_trace_fp32(TraceArgs a)
                 }
             } else {
                 float ox, oy;
-                const int res = finish32(LaneEval<kConfined>{f, dry}, I, s, dtd, dt, kx, ky, ox, oy);
+                const int res = finish32(LaneEval<kConfined, Field32Site>{f, dry}, I, s, dtd, dt, kx,
+                                         ky, ox, oy);
                 // a stage raised: the step is not accepted and the trace ends
                 if (!kConfined && dry)
                     s.status = OKA_TRACE_TRUNCATED;
@@ -207,6 +211,15 @@ k_trace_fp32(TraceArgs a)
     }
 }
 
+// The wells' places relative to the origin, as the FP32 tracer adds them up.
+__global__ void __launch_bounds__(256) k_site_wells32(const double *wells_xy, int nwells, double xo,
+                                                      double yo, float2 *out)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < nwells)
+        out[i] = make_float2((float)(wells_xy[2 * i] - xo), (float)(wells_xy[2 * i + 1] - yo));
+}
+
 // The FP32 tracers' segment rasterizer over the segments of one polyline (one
 // per lane), in coordinates relative to the grid's centre node.
 __global__ void __launch_bounds__(256) k_raster_fp32(RasterArgs a)
@@ -227,11 +240,24 @@ __global__ void __launch_bounds__(256) k_raster_fp32(RasterArgs a)
 
 }  // namespace
 
-size_t trace_fp32_wells_lds(int nwells) { return (size_t)nwells * sizeof(float4); }
+size_t trace_fp32_wells_lds(int nwells, bool confined)
+{
+    return (size_t)((nwells + 3) / 4) * sizeof(float4) * (confined ? 1 : 2);
+}
+
+hipError_t launch_site_wells32(const TraceArgs &a, float2 *out, hipStream_t s)
+{
+    if (a.nwells <= 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(k_site_wells32, dim3((unsigned)((a.nwells + 255) / 256)), dim3(256), 0, s,
+                       a.wells_xy, a.nwells, a.xo, a.yo, out);
+    return hipGetLastError();
+}
 
 hipError_t launch_trace_fp32(const TraceArgs &a, int grid_blocks, int kind, hipStream_t s)
 {
-    size_t lds = trace_fp32_wells_lds(a.nwells) + (a.wmarks ? (size_t)a.w_nr * a.w_nc * 4 : 0);
+    size_t lds = trace_fp32_wells_lds(a.nwells, a.confined) +
+                 (a.wmarks ? (size_t)a.w_nr * a.w_nc * 4 : 0);
     dim3 grid(grid_blocks), block(kTraceBlock);
     if (!a.rasterize || kind == kBmLdsFlat) {
         lds += a.rasterize ? (size_t)a.nwords * 4 : 0;

@@ -35,11 +35,60 @@ constexpr double kInv2Pi = 0.15915494309189535;
 constexpr double kInv4Pi = 0.07957747154594767;
 constexpr double kLn2 = 0.6931471805599453;
 
+// A realization's field, but for its wells, each (xw - xo, yw - yo,
+// q / (2 pi b n), q ln 2 / (4 pi h)), h = K b^2 / 2.
 struct Field32 {
-    const float4 *w;   // (xw - xo, yw - yo, q / (2 pi b n), q ln 2 / (4 pi h)), h = K b^2 / 2
     int nw;
     float a2, b2, c, d, e;  // regional: k_reg = ((a2 dx + c dy) + d, (b2 dy + c dx) + e)
     float pa, pb, pc, pd, pe, pf;   // regional potential over h (unconfined only)
+};
+
+// The field with its wells in LDS, a record each (the pool, whose lanes may be
+// on different sites).
+struct Field32Lds : Field32 {
+    const float4 *w;
+    template <bool kConfined>
+    __device__ __forceinline__ float4 well(int i) const { return w[i]; }
+    template <bool kConfined>
+    __device__ __forceinline__ void wells8(int i, float4 (&r)[8]) const
+    {
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            r[k] = w[i + k];
+    }
+};
+
+// The field of a workgroup that is on one site: the wells' places come by
+// scalar loads from the site's array, and only the strengths are in LDS, read
+// four at a time.  A broadcast LDS read of 16 bytes takes 16 cycles of the
+// CU's LDS, so with a record per well the four SIMDs kept the LDS busy for 64
+// cycles a well, and had 44 of their own to issue: 10^4 x 1000 particles of
+// the 25-well site 39.0 ms against 35.9 ms so (93 VGPRs, 5 waves a SIMD).
+typedef const __attribute__((address_space(4))) float *ConstF32;   // constant: scalar loads
+struct Field32Site : Field32 {
+    ConstF32 xy;                // nw x 2
+    const float4 *q4, *p4;      // LDS, ceil(nw / 4): strengths; the potential's (unconfined)
+    template <bool kConfined>
+    __device__ __forceinline__ float4 well(int i) const
+    {
+        return make_float4(xy[2 * i], xy[2 * i + 1], reinterpret_cast<const float *>(q4)[i],
+                           kConfined ? 0.0f : reinterpret_cast<const float *>(p4)[i]);
+    }
+    template <bool kConfined>
+    __device__ __forceinline__ void wells8(int i, float4 (&r)[8]) const   // i a multiple of 8
+    {
+        const float4 a = q4[i >> 2], b = q4[(i >> 2) + 1];
+        const float q[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        float p[8] = {};
+        if constexpr (!kConfined) {
+            const float4 c = p4[i >> 2], d = p4[(i >> 2) + 1];
+            p[0] = c.x, p[1] = c.y, p[2] = c.z, p[3] = c.w;
+            p[4] = d.x, p[5] = d.y, p[6] = d.z, p[7] = d.w;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            r[k] = make_float4(xy[2 * (i + k)], xy[2 * (i + k) + 1], q[k], p[k]);
+    }
 };
 
 __device__ __forceinline__ void well_term(const float4 &w, float x, float y, float &vx, float &vy)
@@ -66,9 +115,9 @@ __device__ __forceinline__ void well_term_pot(const float4 &w, float x, float y,
     ph = fmaf(w.w, __builtin_amdgcn_logf(r2), ph);
 }
 
-// k = -V at (x, y).  Wells are summed in index order; their LDS reads are
+// k = -V at (x, y).  Wells are summed in index order; their loads are
 // issued 8 at a time so that one trace alone (a long trace after its
-// realization's others ended) does not wait a full LDS round trip per well.
+// realization's others ended) does not wait a full round trip per well.
 //
 // Unconfined (kConfined false), with phi = potential / h (model.py:207-266):
 //   - phi <= 0: the reference raises AquiferError (model.py:342-343); `dry`
@@ -77,8 +126,8 @@ __device__ __forceinline__ void well_term_pot(const float4 &w, float x, float y,
 //     n) is the confined velocity times 1 / sqrt(phi) (model.py:344-345, 384-386);
 //   - otherwise head = (potential + h) / (K b) >= b and V = Q / (b n), the
 //     confined velocity (model.py:346-348, 381-383).
-template <bool kConfined = true>
-__device__ __forceinline__ void feval32(const Field32 &f, float x, float y, float &kx, float &ky,
+template <bool kConfined, class F>
+__device__ __forceinline__ void feval32(const F &f, float x, float y, float &kx, float &ky,
                                         bool &dry)
 {
     float vx = fmaf(f.a2, x, fmaf(f.c, y, f.d));
@@ -87,9 +136,7 @@ __device__ __forceinline__ void feval32(const Field32 &f, float x, float y, floa
     int i = 0;
     for (; i + 8 <= f.nw; i += 8) {
         float4 w[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-            w[k] = f.w[i + k];
+        f.template wells8<kConfined>(i, w);
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             if constexpr (kConfined)
@@ -99,10 +146,11 @@ __device__ __forceinline__ void feval32(const Field32 &f, float x, float y, floa
         }
     }
     for (; i < f.nw; ++i) {
+        const float4 w = f.template well<kConfined>(i);
         if constexpr (kConfined)
-            well_term(f.w[i], x, y, vx, vy);
+            well_term(w, x, y, vx, vy);
         else
-            well_term_pot(f.w[i], x, y, vx, vy, ph);
+            well_term_pot(w, x, y, vx, vy, ph);
     }
     if constexpr (!kConfined) {
         ph += fmaf(fmaf(f.pa, x, fmaf(f.pc, y, f.pd)), x, fmaf(fmaf(f.pb, y, f.pe), y, f.pf));
@@ -117,13 +165,6 @@ __device__ __forceinline__ void feval32(const Field32 &f, float x, float y, floa
     }
     kx = vx;
     ky = vy;
-}
-
-template <bool kConfined = true>
-__device__ __forceinline__ void feval32(const Field32 &f, float x, float y, float &kx, float &ky)
-{
-    bool dry = false;
-    feval32<kConfined>(f, x, y, kx, ky, dry);
 }
 
 // Far wells as local expansions (the FP32 pool on sites of many wells).  The
@@ -244,7 +285,7 @@ __device__ __forceinline__ void near_terms(const float4 *w, VecI4 n, float x, fl
 // coefficients and the first four words of its near row (the count and three
 // indices) are loaded together, and each next four indices while the current
 // four are summed.
-__device__ __forceinline__ bool feval32_far(const Field32 &f, const FarField &F, float x, float y,
+__device__ __forceinline__ bool feval32_far(const Field32Lds &f, const FarField &F, float x, float y,
                                             float &kx, float &ky)
 {
     const float fx = (x - F.x0) * F.ilen, fy = (y - F.y0) * F.ilen;
@@ -288,20 +329,21 @@ __device__ __forceinline__ bool feval32_far(const Field32 &f, const FarField &F,
 // The confined field through the far-well expansions where the point lies
 // in a box, directly elsewhere, as finish32's evaluator.
 struct LaneEvalFar {
-    const Field32 &f;
+    const Field32Lds &f;
     const FarField &F;
     __device__ __forceinline__ void operator()(float x, float y, float &kx, float &ky) const
     {
+        bool dry;
         if (!feval32_far(f, F, x, y, kx, ky))
-            feval32<true>(f, x, y, kx, ky);
+            feval32<true>(f, x, y, kx, ky, dry);
     }
 };
 
 // The lane's own field evaluation, as finish32's evaluator; `dry` collects the
 // unconfined field's AquiferError.
-template <bool kConfined = true>
+template <bool kConfined, class F>
 struct LaneEval {
-    const Field32 &f;
+    const F &f;
     bool &dry;
     __device__ __forceinline__ void operator()(float x, float y, float &kx, float &ky) const
     {

@@ -134,9 +134,9 @@ struct PoolFP32 {
         return I;
     }
 
-    __device__ static Field32 field(const Consts &k, const float4 *w, int nw, bool confined)
+    __device__ static Field32Lds field(const Consts &k, const float4 *w, int nw, bool confined)
     {
-        Field32 f;
+        Field32Lds f;
         f.w = w;
         f.nw = nw;
         f.a2 = k.a2;
@@ -176,7 +176,7 @@ struct PoolFP32 {
     __device__ static int advance(Lane &ln, const Consts &k, const float4 *w, int nw,
                                   PoolBits &bits, bool raster)
     {
-        const Field32 f = field(k, w, nw, kConfined);
+        const Field32Lds f = field(k, w, nw, kConfined);
         const Integ32 I = integ(k);
         double dtd;
         float dt, px, py, kx, ky;
@@ -197,7 +197,7 @@ struct PoolFP32 {
         }
         float ox, oy;
         const int res = far ? finish32(LaneEvalFar{f, k.far}, I, ln.tr, dtd, dt, kx, ky, ox, oy)
-                            : finish32(LaneEval<kConfined>{f, dry}, I, ln.tr, dtd, dt, kx, ky, ox,
+                            : finish32(LaneEval<kConfined, Field32Lds>{f, dry}, I, ln.tr, dtd, dt, kx, ky, ox,
                                        oy);
         // a stage raised: the step is not accepted and the trace ends
         if (!kConfined && dry)

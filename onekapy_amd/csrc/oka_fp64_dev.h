@@ -356,6 +356,72 @@ struct Trace64 {
     int status;
 };
 
+// pow_fifth(x), by a shorter way that gives the same bits: w ~ u^(-1/5) from
+// the hardware's base-2 logarithm and exponential (relative error below 2^-18)
+// and one third-order step (then below 2^-52), y = u w^4, and pow_fifth's own
+// double-double Newton step, with w^4 in place of its division.  x^(0.2 - 1/5)
+// = 1 + t takes a logarithm good to 2^-20.  The sum hi + lo is within 2^-75 of
+// the power, so it decides the rounding unless the two ends of hi + lo
+// (1 +- 2^-70) round apart (once in some 10^5 calls), or x is not an ordinary
+// number: pow_fifth then decides.  A third of its instructions, and no
+// division.  With step_factor, 10^4 x 1000 particles of the 25-well site 131.2
+// -> 126.2 ms, 100 x 100 of the 4-well site (whose lone traces wait for the
+// chain) 9 % less.
+__device__ __forceinline__ double pow_fifth_fast(double x)
+{
+    if (x >= 0x1p-900 && x <= 0x1p900) {
+        int e;
+        const double m = split_exponent(x, &e);
+        const int q = (e + 1000) / 5 - 200;
+        const int r = e - 5 * q;                              // 0..4
+        const double u = m * (double)(1 << r);                // exact, in [1, 32)
+        const float lm = __builtin_amdgcn_logf((float)m);     // base 2
+        double w = (double)__builtin_amdgcn_exp2f(-0.2f * (lm + (float)r));
+        double w2 = w * w;
+        double w4 = w2 * w2;
+        const double d = fma_(-u, w4 * w, 1.0);
+        w = fma_(w, d * fma_(0.12, d, 0.2), w);
+        w2 = w * w;
+        w4 = w2 * w2;
+        const double y = u * w4;
+        const dd y2 = two_prod(y, y);
+        const dd y4 = dd_mul(y2, y2);
+        const dd y5 = dd_mul_d(y4, y);
+        dd rho = two_sum(u, -y5.hi);
+        rho.lo = rho.lo - y5.lo;
+        const double dy = (rho.hi + rho.lo) * (0.2 * w4);
+        const dd root = fast_two_sum(y, dy);
+        const double t = 0x1.999999999999ap-57 * (((double)e + (double)lm) * OKA_LN2_HI);
+        const double lo = root.lo + root.hi * t;
+        const double err = root.hi * 0x1p-70;
+        const double a = root.hi + (lo - err), b = root.hi + (lo + err);
+        if (a == b)
+            return a * pow2i(q);
+    }
+    return pow_fifth(x);
+}
+
+// The step factor min(pow(tol / (est + EPS), 0.2), maxstep / (ds + EPS), 10)
+// of capturezone.py:243-247, as its comparisons give it.  Where the power is
+// certainly above the lesser of the other two, tol > (est + EPS) c^5 (1 +
+// 2^-30) with c^5 in double, it is not evaluated: away from wells the length
+// of the step decides.
+__device__ __forceinline__ double step_factor(double tol, double maxstep, double est, double ds)
+{
+    const double c2 = maxstep / (ds + kEps);
+    double c = c2 < 10.0 ? c2 : 10.0;
+    const double p2 = c * c, p5 = (p2 * p2) * c;
+    const bool above = tol >= 0x1p-500 && ((est + kEps) * p5) * (1.0 + 0x1p-30) < tol;
+    if (!above) {
+        c = pow_fifth_fast(tol / (est + kEps));
+        if (c2 < c)
+            c = c2;
+        if (10.0 < c)
+            c = 10.0;
+    }
+    return c;
+}
+
 // Opens a trace at (xs, ys) (capturezone.py:211-217).  Its k1 = f(start) is
 // the next advance64's evaluation.
 __device__ __forceinline__ void open64(Trace64 &s, const Integ &I, double xs, double ys)
@@ -467,12 +533,7 @@ __device__ __forceinline__ int advance64(const F &f, const Integ &I, Trace64 &s,
         s.by1 = k.yn > s.by1 ? k.yn : s.by1;
         res = 1;
     }
-    double c = pow_fifth(I.tol / (est + kEps));
-    const double c2 = I.maxstep / (ds + kEps);
-    if (c2 < c)
-        c = c2;
-    if (10.0 < c)
-        c = 10.0;
+    const double c = step_factor(I.tol, I.maxstep, est, ds);
     dt = (0.9 * c) * dt;
     s.dt = dt;
     if (fabs(s.t) < I.absdur) {

@@ -5,8 +5,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from onekapy_amd import Realizations, _lib, chronicle_into_field, trace_vertices
-from onekapy_amd.sites import fixed_field
+from onekapy_amd import Realizations, trace_vertices
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +49,21 @@ def test_short_division_rules_bit_exact_vs_oracle(gpu_ctx, case):
     assert (status[0], nverts[0]) == (res.status, res.nverts)
     assert np.array_equal(verts[0, :nverts[0]], ov)
     assert np.array_equal(np.signbit(verts[0, :nverts[0]]), np.signbit(ov))
+
+
+@pytest.mark.parametrize("tol,maxstep", [(1e-9, 10.0), (1e-4, 3.0), (0.02, 1e4), (1e-300, 1.0),
+                                         (1.0, 1e-3)])
+def test_step_factor_rules_bit_exact_vs_oracle(gpu_ctx, tol, maxstep):
+    """The step factor by the power (a tight tolerance), by the step length
+    (a short maxstep) and on either side of the rule between them."""
+    w = np.array([(0.0, 0.0, 0.25, 700.0), (150.0, 80.0, 0.25, 400.0), (-90.0, 60.0, 0.25, -300.0)])
+    real = Realizations([10.0], [0.25], [20.0], w[:, 3].reshape(1, -1), np.array(COEF, float))
+    om = O.OracleModel(0.0, 10.0, 0.25, 20.0, w, 0.0, 0.0, COEF)
+    cap = 1500
+    for start in ((1.25, 0.5), (149.0, 80.5), (-90.0, 61.0)):
+        verts, nverts, status = trace_vertices(np.ascontiguousarray(w[:, :2]), 0.0, 0.0, real,
+                                               np.array([start]), 2000.0, tol, maxstep, True, cap)
+        ov, res = om.backtrace(start[0], start[1], 2000.0, tol, maxstep, confined=True,
+                               max_steps=cap)
+        assert (status[0], nverts[0]) == (res.status, res.nverts)
+        assert np.array_equal(verts[0, :nverts[0]], ov)

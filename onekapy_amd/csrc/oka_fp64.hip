@@ -92,8 +92,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
     const int tid = threadIdx.x;
     const int P = a.npaths;
     const Integ I = make_integ(a);
-    const double umbra = a.umbra;
-    const double u2 = umbra * umbra;
+    const Raster64 rk = make_raster(a.gdx, a.gdy, a.umbra, grid_extent(a));
     const bool raster = !kVerts && a.rasterize;
     uint32_t *lds_tail = reinterpret_cast<uint32_t *>(s_nq + a.nwells);
     Chron<kMode> ch;
@@ -161,8 +160,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
             const int res = advance64<kConfined>(f, I, s, fresh, ox, oy);
             if (res & 1) {
                 if (raster)
-                    n_cand += (unsigned long long)raster_segment(ch.bits, ep, a.gdx, a.gdy, umbra,
-                                                                 u2, ox, oy, s.x, s.y);
+                    n_cand += (unsigned long long)raster_segment(ch.bits, ep, rk, ox, oy, s.x, s.y);
                 if (kVerts && s.acc < a.vcap) {
                     a.verts[2 * (k * a.vcap + s.acc)] = s.x;
                     a.verts[2 * (k * a.vcap + s.acc) + 1] = s.y;
@@ -304,7 +302,9 @@ __global__ void __launch_bounds__(256) k_raster_fp64(RasterArgs a)
         return;
     EpochReg e{a.xmin, a.ymin, a.nrows, a.ncols, 0, 0};
     FlatBits bits{a.bitmap, a.ncols};
-    raster_segment(bits, e, a.dx, a.dy, a.umbra, a.umbra * a.umbra, a.xy[2 * i], a.xy[2 * i + 1],
+    const double gmax = fmax(fmax(fabs(a.xmin), fabs(a.xmin + a.ncols * a.dx)),
+                             fmax(fabs(a.ymin), fabs(a.ymin + a.nrows * a.dy)));
+    raster_segment(bits, e, make_raster(a.dx, a.dy, a.umbra, gmax), a.xy[2 * i], a.xy[2 * i + 1],
                    a.xy[2 * i + 2], a.xy[2 * i + 3]);
 }
 

@@ -569,19 +569,100 @@ __device__ __forceinline__ EpochReg find_epoch(const TraceArgs &a, int64_t k)
     return {e.xmin, e.ymin, e.nrows, e.ncols, e.row_off, e.col_off};
 }
 
-// probabilityfield.py:292-310 for one segment, marking nodes of the final grid
-// in `bits` (FlatBits or TileBits).  Already-marked nodes are skipped, as the
-// reference does.
+// The rasterizer's constants: the lattice spacing with its reciprocals and
+// the umbra; the rest serve the outer chords of raster_segment, in float.
+struct Raster64 {
+    double dx, dy, rdx, rdy, umbra, u2;
+    float idx, fdy, slack, outer, outer2;   // 1 / dx, dy; 2^-10 umbra; umbra + slack; its square
+    int fast;                               // the chords and the short quotients apply
+};
+
+// gmax: the largest magnitude of the lattice's coordinates.
+__device__ __forceinline__ Raster64 make_raster(double dx, double dy, double umbra, double gmax)
+{
+    Raster64 g;
+    g.dx = dx;
+    g.dy = dy;
+    g.rdx = recip_plain(dx);
+    g.rdy = recip_plain(dy);
+    g.umbra = umbra;
+    g.u2 = umbra * umbra;
+    g.idx = (float)g.rdx;
+    g.fdy = (float)dy;
+    g.slack = (float)umbra * 0x1p-10f;
+    g.outer = (float)umbra + g.slack;
+    g.outer2 = g.outer * g.outer;
+    // float range; the window at most 1,000 umbras per spacing; the rounding
+    // of the coordinates far below the slack
+    g.fast = umbra >= 1e-12 && umbra <= 1e12 && dx <= 1e3 * umbra && dy <= 1e3 * umbra &&
+             dx >= 1e-6 * umbra && dy >= 1e-6 * umbra && gmax <= 0x1p36 * umbra;
+    return g;
+}
+
+__device__ __forceinline__ double grid_extent(const TraceArgs &a)
+{
+    return fmax(fmax(fabs(a.gxmin), fabs(a.gxmax)), fmax(fabs(a.gymin), fabs(a.gymax)));
+}
+
+// probabilityfield.py:296-310, 407-427 for one node (row, col of the final
+// grid; j, i of the epoch's): marks it if it is strictly within umbra.
 template <typename Bits>
-__device__ __forceinline__ int raster_segment(Bits &bits, const EpochReg &e, double dx, double dy,
-                                               double umbra, double u2, double ax, double ay,
-                                               double bx, double by)
+__device__ __forceinline__ void raster_node(Bits &bits, const EpochReg &e, const Raster64 &g,
+                                            double ax, double ay, double bax, double bay, double l2,
+                                            int i, int j)
+{
+    const double cx = e.xmin + (double)j * g.dx;
+    const double cax = cx - ax;
+    const double cy = e.ymin + (double)i * g.dy;
+    const double cay = cy - ay;
+    const double perp = bax * cay - bay * cax;
+    const double dot = bax * cax + bay * cay;
+    double al, be;
+    div_pair(perp * perp, dot * dot, l2, al, be);
+    double d2;
+    if (dot < 0.0)
+        d2 = al + be;
+    else if (be > l2)
+        d2 = ((al + be) - 2.0 * dot) + l2;
+    else
+        d2 = al;
+    if (d2 < g.u2)
+        bits.set(i + e.roff, j + e.coff);
+}
+
+// probabilityfield.py:292-310 for one segment, marking nodes of the final grid
+// in `bits` (FlatBits, TileBits or PoolBits).  Already-marked nodes are
+// skipped, as the reference does.  Returns the size of the reference's
+// candidate window.
+//
+// Most of a window's nodes lie outside the umbra or are marked already, so
+// each row first takes, in float, the chord of the capsule around the segment
+// at a radius 2^-10 larger than umbra (raster32's, with its clip widened by as
+// much), which contains every node the exact test could mark: the float
+// errors are below 2^-20 of the umbra for segments up to 1,000 umbras.  Only
+// its unmarked nodes, read a word at a time, take the exact test.  Against the
+// exact test at every unmarked node of the window: 10^4 x 1000 particles of
+// the 25-well site 126.2 -> 119.9 ms, 100 x 100 of the 4-well site 14 % less.
+template <typename Bits>
+__device__ __forceinline__ int raster_segment(Bits &bits, const EpochReg &e, const Raster64 &g,
+                                               double ax, double ay, double bx, double by)
 {
     const double lox = bx < ax ? bx : ax, hix = bx > ax ? bx : ax;
     const double loy = by < ay ? by : ay, hiy = by > ay ? by : ay;
+    const double nxl = (lox - g.umbra) - e.xmin, nxr = (hix + g.umbra) - e.xmin;
+    const double nyl = (loy - g.umbra) - e.ymin, nyr = (hiy + g.umbra) - e.ymin;
     double qxl, qxr, qyl, qyr;
-    div_pair((lox - umbra) - e.xmin, (hix + umbra) - e.xmin, dx, qxl, qxr);
-    div_pair((loy - umbra) - e.ymin, (hiy + umbra) - e.ymin, dy, qyl, qyr);
+    const bool plain = g.fast && fmin(fmin(fabs(nxl), fabs(nxr)), fmin(fabs(nyl), fabs(nyr))) >= 0x1p-300 &&
+                       fmax(fmax(fabs(nxl), fabs(nxr)), fmax(fabs(nyl), fabs(nyr))) <= 0x1p300;
+    if (__ballot(!plain) == 0ull) {
+        qxl = quot_plain(nxl, g.dx, g.rdx);
+        qxr = quot_plain(nxr, g.dx, g.rdx);
+        qyl = quot_plain(nyl, g.dy, g.rdy);
+        qyr = quot_plain(nyr, g.dy, g.rdy);
+    } else {
+        div_pair(nxl, nxr, g.dx, qxl, qxr);
+        div_pair(nyl, nyr, g.dy, qyl, qyr);
+    }
     double jl = floor(qxl);
     double jr = floor(qxr) + 1.0;
     double il = floor(qyl);
@@ -595,32 +676,61 @@ __device__ __forceinline__ int raster_segment(Bits &bits, const EpochReg &e, dou
     const int j0 = (int)jl, j1 = (int)jr, i0 = (int)il, i1 = (int)ir;
     const double bax = bx - ax, bay = by - ay;
     const double l2 = bax * bax + bay * bay;
-    for (int j = j0; j < j1; ++j) {
-        const double cx = e.xmin + (double)j * dx;
-        const double cax = cx - ax;
-        const int col = j + e.coff;
-        for (int i = i0; i < i1; ++i) {
-            const int row = i + e.roff;
-            if (bits.test(row, col))
+    const int ncand = (j1 - j0) * (i1 - i0);
+    // the row's chord: x - ax in (lo, hi) with c = y_row - ay; in columns from j0
+    const float fbx = (float)bax, fby = (float)bay, fl2 = (float)l2;
+    const bool chord = g.fast && fabsf(fbx) > 1e-20f && fabsf(fby) > 1e-20f &&
+                       fl2 < 1e6f * g.outer2 && j1 - j0 < 4096 && i1 - i0 < 4096;
+    const float ibx = __builtin_amdgcn_rcpf(fbx), iby = __builtin_amdgcn_rcpf(fby);
+    const float len = __builtin_amdgcn_sqrtf(fl2);
+    const float kb = -fby * ibx, ka = fbx * iby;
+    const float clip = g.slack * len * fabsf(ibx), l2b = fl2 * ibx;
+    const float blo = fminf(l2b, 0.0f) - clip, bhi = fmaxf(l2b, 0.0f) + clip;
+    const float wr = g.outer * len * fabsf(iby);
+    const float xa = (float)((ax - (e.xmin + jl * g.dx)) * g.rdx);   // A's column from j0
+    const float c0 = (float)((e.ymin + il * g.dy) - ay);
+    const float last = (float)(j1 - j0 - 1);
+    for (int i = i0; i < i1; ++i) {
+        int ja = j0, jb = j1 - 1;
+        if (chord) {
+            const float c = fmaf((float)(i - i0), g.fdy, c0);
+            float lo = fmaxf(fmaf(kb, c, blo), fmaf(ka, c, -wr));
+            float hi = fminf(fmaf(kb, c, bhi), fmaf(ka, c, wr));
+            if (!(lo < hi)) {
+                lo = INFINITY;
+                hi = -INFINITY;
+            }
+            const float ha = fmaf(-c, c, g.outer2);
+            if (ha > 0.0f) {
+                const float r = __builtin_amdgcn_sqrtf(ha);
+                lo = fminf(lo, -r);
+                hi = fmaxf(hi, r);
+            }
+            const float cb = c - fby;
+            const float hb = fmaf(-cb, cb, g.outer2);
+            if (hb > 0.0f) {
+                const float r = __builtin_amdgcn_sqrtf(hb);
+                lo = fminf(lo, fbx - r);
+                hi = fmaxf(hi, fbx + r);
+            }
+            const float fa = fmaxf(ceilf(fmaf(lo, g.idx, xa - 0x1p-8f)), 0.0f);
+            const float fb = fminf(floorf(fmaf(hi, g.idx, xa + 0x1p-8f)), last);
+            if (!(fa <= fb))
                 continue;
-            const double cy = e.ymin + (double)i * dy;
-            const double cay = cy - ay;
-            const double perp = bax * cay - bay * cax;
-            const double dot = bax * cax + bay * cay;
-            double al, be;
-            div_pair(perp * perp, dot * dot, l2, al, be);
-            double d2;
-            if (dot < 0.0)
-                d2 = al + be;
-            else if (be > l2)
-                d2 = ((al + be) - 2.0 * dot) + l2;
-            else
-                d2 = al;
-            if (d2 < u2)
-                bits.set(row, col);
+            ja = j0 + (int)fa;
+            jb = j0 + (int)fb;
+        }
+        for (; ja <= jb; ja += 32) {
+            const int n = min(jb - ja + 1, 32);
+            uint32_t todo = ~bits.window(i + e.roff, ja + e.coff, n) & span_mask(n, 0);
+            while (todo) {
+                const int k = __ffs(todo) - 1;
+                todo &= todo - 1u;
+                raster_node(bits, e, g, ax, ay, bax, bay, l2, i, ja + k);
+            }
         }
     }
-    return (j1 - j0) * (i1 - i0);
+    return ncand;
 }
 
 __device__ __forceinline__ Integ make_integ(const TraceArgs &a)

@@ -149,6 +149,15 @@ struct FlatBits {
         const int idx = row * ncols + col;
         atomicOr(&bm[idx >> 5], 1u << (idx & 31));
     }
+    // Bit k of the result: column c0 + k of the row is marked (1 <= n <= 32).
+    __device__ __forceinline__ uint32_t window(int row, int c0, int n) const
+    {
+        const int idx = row * ncols + c0, b = idx & 31;
+        uint64_t v = bm[idx >> 5];
+        if (b + n > 32)
+            v |= (uint64_t)bm[(idx >> 5) + 1] << 32;
+        return (uint32_t)(v >> b) & span_mask(n, 0);
+    }
     // Row stride of the flat index (the span markers' `base` = row * stride).
     __device__ __forceinline__ int stride() const { return ncols; }
     // Marks columns c0..c1 (inclusive) of one row, whose first node has flat
@@ -195,6 +204,17 @@ struct TileBits {
     {
         const uint32_t *w = word((row >> 5) * tiles_x + (col >> 5), row & 31);
         return w != nullptr && ((*w >> (col & 31)) & 1u);
+    }
+    __device__ __forceinline__ uint32_t window(int row, int c0, int n) const
+    {
+        const int t = (row >> 5) * tiles_x + (c0 >> 5), b = c0 & 31;
+        const uint32_t *w = word(t, row & 31);
+        uint64_t v = w ? *w : 0u;
+        if (b + n > 32) {
+            w = word(t + 1, row & 31);
+            v |= (uint64_t)(w ? *w : 0u) << 32;
+        }
+        return (uint32_t)(v >> b) & span_mask(n, 0);
     }
     // The first lane to claim a tile maps it; a lane that loses the race uses
     // the winner's slot, and its own slot stays unmapped (and zero).

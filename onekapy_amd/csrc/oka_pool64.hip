@@ -23,7 +23,7 @@ struct PoolFP64 {
     struct Consts {
         double xo, yo, A, B, C, D, E, F, A2, B2, K, bt, bn, rbn, por, half_kb2;   // Field64
         double dur, absdur, tol, maxstep, sg;                               // Integ
-        double gdx, gdy, umbra, u2;
+        Raster64 raster;
         long long cap;
         int plain, pad[3];
     };
@@ -82,10 +82,7 @@ struct PoolFP64 {
         k.sg = A.duration > 0.0 ? 1.0
                                 : (A.duration < 0.0 ? -1.0 : (A.duration == 0.0 ? 0.0 : (double)NAN));
         k.cap = A.max_steps;
-        k.gdx = A.gdx;
-        k.gdy = A.gdy;
-        k.umbra = A.umbra;
-        k.u2 = A.umbra * A.umbra;
+        k.raster = make_raster(A.gdx, A.gdy, A.umbra, grid_extent(A));
         k.rbn = recip_plain(k.bn);
         k.plain = plain_field(field(k, nullptr, 0)) ? plain : kPlainNever;
     }
@@ -156,8 +153,8 @@ struct PoolFP64 {
         if ((res & 1) && raster) {
             bits.last_t = ln.last_t;
             bits.last_v = ln.last_v;
-            ln.cand += (unsigned long long)raster_segment(bits, ln.ep, k.gdx, k.gdy, k.umbra, k.u2,
-                                                          ox, oy, ln.s.x, ln.s.y);
+            ln.cand += (unsigned long long)raster_segment(bits, ln.ep, k.raster, ox, oy, ln.s.x,
+                                                           ln.s.y);
             ln.last_t = bits.last_t;
             ln.last_v = bits.last_v;
         }

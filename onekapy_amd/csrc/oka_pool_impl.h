@@ -149,16 +149,30 @@ struct PoolBits {
         }
         return v;
     }
-    __device__ __forceinline__ bool test(int row, int col)
+    // The word of tile t's row r (0 when the tile is unmapped).
+    __device__ __forceinline__ uint32_t row_word(uint32_t t, int r)
     {
-        const uint32_t t = (uint32_t)((row >> 5) * tiles_x + (col >> 5));
         uint32_t v = lookup(t);
         if (v == kValNone) {
             if (!__hip_atomic_load(hash_full, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
-                return false;
+                return 0u;
             v = kValHbm;
         }
-        return (tile_words(t, v)[row & 31] >> (col & 31)) & 1u;
+        return tile_words(t, v)[r];
+    }
+    __device__ __forceinline__ bool test(int row, int col)
+    {
+        return (row_word((uint32_t)((row >> 5) * tiles_x + (col >> 5)), row & 31) >> (col & 31)) & 1u;
+    }
+    // Bit k of the result: column c0 + k of the row is marked (1 <= n <= 32).
+    __device__ __forceinline__ uint32_t window(int row, int c0, int n)
+    {
+        const uint32_t t = (uint32_t)((row >> 5) * tiles_x + (c0 >> 5));
+        const int b = c0 & 31;
+        uint64_t v = row_word(t, row & 31);
+        if (b + n > 32)
+            v |= (uint64_t)row_word(t + 1, row & 31) << 32;
+        return (uint32_t)(v >> b) & span_mask(n, 0);
     }
     __device__ __forceinline__ void set(int row, int col)
     {

@@ -5,12 +5,11 @@ the decile loop of oneka/oneka.py:279-288).
 
 pr lists every node's Pr(capture) = pgrid / total_weight in descending order
 and area[i] = (i + 1) * spacing^2 is the area where Pr(capture) >= pr[i].
-With weight 1 per realization (stochastic.py:265) pgrid holds integer counts
-k, so pr takes the values k / total_weight and the descending sort is a
-counting sort: the GPU histogram of the counts (oka_count_histogram) gives the
-same array as numpy's sort, value for value.  Any other field (weights other
-than 1, e.g. compute_capturezone's weight argument) is sorted on the GPU by a
-radix sort of the probabilities (oka_field_sorted_probabilities).
+The GPU sorts the probabilities (oka_field_sorted_probabilities): with weight 1
+per realization (stochastic.py:265) pgrid holds integer counts and the sort is
+a counting sort, any other field (weights other than 1, e.g.
+compute_capturezone's weight argument) is radix-sorted; both give the same
+array as numpy's sort, value for value.
 """
 import math
 
@@ -49,17 +48,9 @@ def impact_curve(spacing, pf):
     """(pr, area) as create_impact_plot returns them (visualize.py:382-385)."""
     if pf.total_weight <= 0:
         raise CaptureZoneError('Empty capture zone')
-    counts = np.rint(pf.pgrid)
-    if np.array_equal(counts, pf.pgrid) and counts.min(initial=0) >= 0 and \
-            counts.max(initial=0) < 2 ** 31:
-        top = int(counts.max(initial=0))
-        hist = count_histogram(counts.astype(np.int32), top)
-        values = np.arange(top, -1, -1, dtype=np.float64) / pf.total_weight   # descending
-        pr = np.repeat(values, hist[::-1])
-    else:
-        pr = sorted_probabilities(pf.pgrid, pf.total_weight)
-    n = pr.shape[0]
-    area = (np.arange(n) + 1) * spacing ** 2
+    pr = sorted_probabilities(pf.pgrid, pf.total_weight)
+    area = np.arange(1.0, pr.shape[0] + 1.0)
+    area *= spacing ** 2
     return pr, area
 
 

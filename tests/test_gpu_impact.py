@@ -98,3 +98,19 @@ def test_smoothed_probability_equals_scipy(gpu_ctx, smooth):
         assert np.array_equal(got, want)
     with pytest.raises(CaptureZoneError):
         smoothed_probability(_field(ref["counts"], 0.0), smooth)
+
+
+@pytest.mark.parametrize("top,n", [(0, 1), (1, 255), (3, 4096), (1024, 70001), (131072, 5000),
+                                   (131073, 5000), (10, 600000)])
+def test_sorted_counts_equal_numpy_on_both_routes(gpu_ctx, top, n):
+    """Whole counts up to 2^17 are sorted by counting, larger ones (and any
+    other value among them) by the radix sort; both equal numpy's sort."""
+    rng = np.random.default_rng(top + n)
+    g = rng.integers(0, top + 1, n).astype(np.float64)
+    g[rng.random(n) < 0.5] = 0.0
+    g[rng.integers(0, n)] = float(top)
+    for total in (7.0, 0.3):
+        assert np.array_equal(sorted_probabilities(g, total), np.flip(np.sort(g / total)))
+    for odd in (0.5, -1.0, -0.0, 1e300, np.inf):
+        g[n // 2] = odd
+        assert np.array_equal(sorted_probabilities(g, 7.0), np.flip(np.sort(g / 7.0)))

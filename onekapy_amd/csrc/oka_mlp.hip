@@ -434,7 +434,7 @@ k_gemm_accum(GemmArgs g, int rt)
     __syncthreads();
     if (threadIdx.x < S::BN) {
         const int n = ct * S::BN + threadIdx.x;
-        // the workgroup's rows (at most 8 x 128) lie in one row of the sums
+        // the workgroup's rows (at most 4 x 128) lie in one row of the sums
         const int64_t sr = g.sum_rows ? (g.sum_row0 + (int64_t)rg * rt * S::BM) / g.sum_rows : 0;
         atomicAdd(&g.sums[sr * g.N + n], (double)sm.col[0][threadIdx.x]);
         if (g.sums_sq)
@@ -671,7 +671,12 @@ __global__ void k_zero_f64(double *p, int64_t n)
 using namespace mlp;
 
 // 128 x 128 tiles when every product of the launch divides into them and
-// they still give the GPU at least one workgroup per CU; 64 x 64 otherwise.
+// they still give each CU two workgroups, of which one computes while the
+// other waits at a barrier or in its epilogue; 64 x 64 otherwise (the hidden
+// layers of 8,192 rows: 256 big tiles, 16 us; 1,024 small ones, 9 us).  A dW
+// product beside its dX takes them from one workgroup per CU on: its K is
+// long, and split plans raise the count (dW3 with dX3 at batch 2,048: 32 us
+// big, 47 small).
 static bool use_big_tiles(const GemmArgs &g1, const GemmArgs *g2)
 {
     // compute units of the current device (the caller has set it)
@@ -683,7 +688,7 @@ static bool use_big_tiles(const GemmArgs &g1, const GemmArgs *g2)
     auto fits = [](const GemmArgs &g) { return g.M % 128 == 0 && g.N % 128 == 0; };
     if (!fits(g1) || (g2 && !fits(*g2)))
         return false;
-    return gemm_tiles(g1, 1) + (g2 ? gemm_tiles(*g2, 1) : 0) >= num_cu;
+    return gemm_tiles(g1, 1) + (g2 ? gemm_tiles(*g2, 1) : 0) >= (g2 ? 1 : 2) * num_cu;
 }
 
 int gemm2_workgroups(const GemmArgs &g1, const GemmArgs *g2)
@@ -701,7 +706,9 @@ hipError_t launch_gemm2(int e1, const GemmArgs &g1, int e2, const GemmArgs &g2, 
         return hipErrorInvalidValue;
     const bool big = use_big_tiles(g1, e2 == kEpiNone ? nullptr : &g2);
     if (e1 == kEpiAccum && e2 == kEpiNone) {
-        constexpr int kRowTiles = 8;
+        // 4 row tiles a workgroup: 2 workgroups per CU at 8,192 rows of 4,096
+        // outputs (66 us; 86 with 8 row tiles, one workgroup per CU)
+        constexpr int kRowTiles = 4;
         const int bt = big ? 128 : 64;
         const int gy = g1.M / bt;
         const dim3 grid((g1.N / bt) * ((gy + kRowTiles - 1) / kRowTiles));

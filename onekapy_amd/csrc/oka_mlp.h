@@ -48,7 +48,8 @@ struct GemmArgs {
 
 // One FP32 master segment of the parameter vector updated by Adam: a weight
 // matrix [rows, cols] with its BF16 copies (wh row-major, wt transposed), or a
-// bias vector laid out as [len / 32, 32] with wh = wt = nullptr.
+// bias vector laid out as [len / 64, 64] with wh = wt = nullptr; cols a
+// multiple of 64, 16-byte aligned.
 struct AdamSeg {
     int64_t off;
     int rows, cols;

@@ -518,17 +518,24 @@ __global__ void __launch_bounds__(256) k_prep_input(const float *x, int n_in, in
     }
 }
 
-// Adam over one 32 x 32 tile of one segment per workgroup; weight segments
-// also refresh their BF16 copies (the transposed one through LDS so that both
-// stores are coalesced).
+// Adam over one 64 x 64 tile of one segment per workgroup (cols a multiple of
+// 64); weight segments also refresh their BF16 copies, the transposed one
+// through LDS so that both leave as 16-byte row segments.  Memory bound: 6
+// words a parameter, the gradient's slices and 4 bytes of BF16.  Each lane has
+// the 16-byte loads of 4 rows and all their slices in flight before the first
+// is used, and before the bias corrections' double-precision powers.
+// 2.39 M parameters with two slices of W3's gradient: 16.2 us (5.4 TB/s)
+// against 19.3 with 32 x 32 tiles and 4-byte accesses.
+constexpr int kAdamTile = 64;
+
 __global__ void __launch_bounds__(256) k_adam(AdamArgs a)
 {
-    __shared__ uint16_t tile[32][33];
+    __shared__ uint16_t tile[kAdamTile][kAdamTile + 2];   // [column][row]
     __shared__ float corr[2];
     int b = blockIdx.x, s = 0, ct = 1;
     for (; s < a.nseg; ++s) {
-        ct = (a.seg[s].cols + 31) / 32;
-        const int tiles = ct * ((a.seg[s].rows + 31) / 32);
+        ct = a.seg[s].cols / kAdamTile;
+        const int tiles = ct * ((a.seg[s].rows + kAdamTile - 1) / kAdamTile);
         if (b < tiles)
             break;
         b -= tiles;
@@ -536,7 +543,21 @@ __global__ void __launch_bounds__(256) k_adam(AdamArgs a)
     if (s >= a.nseg)
         return;   // the grid is sized to the segments; never taken
     const AdamSeg sg = a.seg[s];
-    const int r0 = (b / ct) * 32, c0 = (b % ct) * 32;
+    const int r0 = (b / ct) * kAdamTile, c0 = (b % ct) * kAdamTile;
+    const int tr = threadIdx.x >> 4, tc = (threadIdx.x & 15) * 4;
+    float4 g[4], m[4], v[4], p[4];
+    auto load = [](const float *src) { return *reinterpret_cast<const float4 *>(src); };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int r = r0 + tr + 16 * k;
+        if (r < sg.rows) {
+            const int64_t e = (int64_t)r * sg.cols + c0 + tc, i = sg.off + e;
+            m[k] = load(a.m + i);
+            v[k] = load(a.v + i);
+            p[k] = load(a.p + i);
+            g[k] = load(sg.nslices > 0 ? sg.slices + e : a.grad + i);
+        }
+    }
     if (threadIdx.x == 0) {
         const int64_t t = a.dstate ? a.tbase + a.dstate[1] : a.tbase;
         // bias corrections 1/(1 - beta^t)
@@ -545,41 +566,66 @@ __global__ void __launch_bounds__(256) k_adam(AdamArgs a)
         if (a.dstate && blockIdx.x == 0)
             a.dstate[0] += 1;   // no kernel of this launch reads dstate[0]
     }
+    const int64_t sz = (int64_t)sg.rows * sg.cols;
+    for (int q = 1; q < sg.nslices; ++q) {   // the slices in order
+        float4 x[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int r = r0 + tr + 16 * k;
+            if (r < sg.rows)
+                x[k] = load(sg.slices + q * sz + (int64_t)r * sg.cols + c0 + tc);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            g[k].x += x[k].x;
+            g[k].y += x[k].y;
+            g[k].z += x[k].z;
+            g[k].w += x[k].w;
+        }
+    }
     __syncthreads();
     const float c1 = corr[0], c2 = corr[1];
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;   // 32 x 8 lanes
-    for (int k = ty; k < 32; k += 8) {
-        const int r = r0 + k, c = c0 + tx;
-        if (r < sg.rows && c < sg.cols) {
-            const int64_t i = sg.off + (int64_t)r * sg.cols + c;
-            float gi;
-            if (sg.nslices > 0) {
-                const int64_t e = (int64_t)r * sg.cols + c, sz = (int64_t)sg.rows * sg.cols;
-                gi = sg.slices[e];
-                for (int k = 1; k < sg.nslices; ++k)
-                    gi += sg.slices[k * sz + e];
-            } else {
-                gi = a.grad[i];
-            }
-            const float mi = a.b1 * a.m[i] + (1.f - a.b1) * gi;
-            const float vi = a.b2 * a.v[i] + (1.f - a.b2) * gi * gi;
-            a.m[i] = mi;
-            a.v[i] = vi;
-            const float pi = a.p[i] - a.lr * (mi * c1) / (sqrtf(vi * c2) + a.eps);
-            a.p[i] = pi;
-            if (sg.wh) {
-                const uint16_t h = f2bf(pi);
-                sg.wh[(int64_t)r * sg.cols + c] = h;
-                tile[k][tx] = h;
-            }
+    auto step = [&](float gi, float &mi, float &vi, float &pi) {
+        mi = a.b1 * mi + (1.f - a.b1) * gi;
+        vi = a.b2 * vi + (1.f - a.b2) * gi * gi;
+        pi = pi - a.lr * (mi * c1) / (sqrtf(vi * c2) + a.eps);
+    };
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int r = r0 + tr + 16 * k;
+        if (r >= sg.rows)
+            continue;
+        step(g[k].x, m[k].x, v[k].x, p[k].x);
+        step(g[k].y, m[k].y, v[k].y, p[k].y);
+        step(g[k].z, m[k].z, v[k].z, p[k].z);
+        step(g[k].w, m[k].w, v[k].w, p[k].w);
+        const int64_t e = (int64_t)r * sg.cols + c0 + tc, i = sg.off + e;
+        *reinterpret_cast<float4 *>(a.m + i) = m[k];
+        *reinterpret_cast<float4 *>(a.v + i) = v[k];
+        *reinterpret_cast<float4 *>(a.p + i) = p[k];
+        if (sg.wh) {
+            const uint16_t h[4] = {f2bf(p[k].x), f2bf(p[k].y), f2bf(p[k].z), f2bf(p[k].w)};
+            uint2 packed;
+            packed.x = (uint32_t)h[0] | ((uint32_t)h[1] << 16);
+            packed.y = (uint32_t)h[2] | ((uint32_t)h[3] << 16);
+            *reinterpret_cast<uint2 *>(sg.wh + e) = packed;
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                tile[tc + j][tr + 16 * k] = h[j];
         }
     }
     if (sg.wh) {
         __syncthreads();
-        for (int k = ty; k < 32; k += 8) {
-            const int c = c0 + k, r = r0 + tx;
-            if (r < sg.rows && c < sg.cols)
-                sg.wt[(int64_t)c * sg.rows + r] = tile[tx][k];
+        // column c of the tile is 64 consecutive values of the transposed copy
+        const int c = threadIdx.x >> 2, rr = (threadIdx.x & 3) * 16;
+        if (r0 + rr < sg.rows) {
+            uint32_t w[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                w[k] = *reinterpret_cast<const uint32_t *>(&tile[c][rr + 2 * k]);
+            uint4 *dst = reinterpret_cast<uint4 *>(sg.wt + (int64_t)(c0 + c) * sg.rows + r0 + rr);
+            dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
+            dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
         }
     }
 }
@@ -768,9 +814,11 @@ hipError_t launch_adam(const AdamArgs &a, hipStream_t s)
 {
     int blocks = 0;
     for (int i = 0; i < a.nseg; ++i) {
-        if (a.seg[i].rows < 1 || a.seg[i].cols < 1)
+        // 16-byte rows; a weight matrix's transposed copy in 16-row pieces
+        if (a.seg[i].rows < 1 || a.seg[i].cols < 1 || a.seg[i].cols % kAdamTile ||
+            (a.seg[i].wh && a.seg[i].rows % 16))
             return hipErrorInvalidValue;
-        blocks += ((a.seg[i].cols + 31) / 32) * ((a.seg[i].rows + 31) / 32);
+        blocks += (a.seg[i].cols / kAdamTile) * ((a.seg[i].rows + kAdamTile - 1) / kAdamTile);
     }
     if (blocks == 0)
         return hipSuccess;

@@ -529,7 +529,7 @@ int oka_mlp_train(oka_mlp *M, int64_t nsamples, const float *x, const uint8_t *m
             const bool sl = split[l] > 1;
             a.seg[2 * l] = AdamSeg{oW[l], rows[l], cols[l], wh[l], wt[l], sl ? M->ws[l] : nullptr,
                                    sl ? split[l] : 0};
-            a.seg[2 * l + 1] = AdamSeg{ob[l], rows[l] / 32, 32, nullptr, nullptr,
+            a.seg[2 * l + 1] = AdamSeg{ob[l], rows[l] / 64, 64, nullptr, nullptr,
                                        sl ? M->bs[l] : nullptr, sl ? split[l] : 0};
         }
         a.nseg = 6;

@@ -258,7 +258,7 @@ hipError_t launch_trace_fp32(const TraceArgs &a, int grid_blocks, int kind, hipS
 {
     size_t lds = trace_fp32_wells_lds(a.nwells, a.confined) +
                  (a.wmarks ? (size_t)a.w_nr * a.w_nc * 4 : 0);
-    dim3 grid(grid_blocks), block(kTraceBlock);
+    dim3 grid(grid_blocks), block(trace_block(a.npaths));
     if (!a.rasterize || kind == kBmLdsFlat) {
         lds += a.rasterize ? (size_t)a.nwords * 4 : 0;
         if (a.confined)

@@ -311,7 +311,7 @@ __global__ void __launch_bounds__(256) k_raster_fp64(RasterArgs a)
 template <int kMode>
 hipError_t launch_mode(const TraceArgs &a, int grid_blocks, size_t lds, hipStream_t s)
 {
-    dim3 grid(grid_blocks), block(kTraceBlock);
+    dim3 grid(grid_blocks), block(trace_block(a.npaths));
     if (a.confined)
         hipLaunchKernelGGL((k_trace_fp64<true, kMode>), grid, block, lds, s, a);
     else

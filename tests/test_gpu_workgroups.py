@@ -1,0 +1,21 @@
+"""The workgroup schedule's launch shapes: whatever lanes a realization's
+particles are given, the counts, per-trace statuses and statistics are those of
+the pool, which deals out particles on its own."""
+import pytest
+
+from onekapy_amd import _lib, sites
+from helpers import oracle_fit_draw, small_site
+from test_gpu_pool import _both
+
+pytestmark = pytest.mark.gpu
+
+
+# a lone particle; a wave and one more; whole waves; the largest workgroup and
+# the first refilled lane
+@pytest.mark.parametrize("npaths", [1, 64, 65, 192, 256, 257])
+@pytest.mark.parametrize("precision", [_lib.FP64_EXACT, _lib.FP32], ids=["fp64", "fp32"])
+def test_lanes_for_the_particles(gpu_ctx, npaths, precision):
+    s, d = small_site(nreal=6, npaths=npaths)
+    _, _, coef = oracle_fit_draw(s, d)
+    print(f"npaths {npaths} precision {precision}", flush=True)
+    _both(s, d, coef, s.fixed_field(), s.umbra, precision)

@@ -478,6 +478,10 @@ int check_opts(oka_ctx *c, const oka_trace_opts *o)
 
 constexpr int64_t kDefaultMaxSteps = 1000000;
 
+// Most memory for the merged bitmaps of shared realizations and the overflow
+// regions beside them.
+constexpr int64_t kMaxShareBytes = 2ll << 30;
+
 // The workgroup schedule takes as many wells as whole records of them (32
 // bytes in FP64, 16 in FP32) fit in a workgroup's LDS.
 size_t wells_limit_lds(int nwells, bool fp64) { return (size_t)nwells * (fp64 ? 32 : 16); }
@@ -1062,30 +1066,58 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
                                 trace_steps, stats, flags, win, marks, masks);
     }
 
-    // launch shape: one realization per 256-lane workgroup, grid-stride
+    // launch shape: a realization per workgroup of up to 256 lanes
     const size_t base_lds =
         (fp64 ? trace_fp64_wells_lds(a.nwells) : trace_fp32_wells_lds(a.nwells, a.confined)) +
         win_lds;
     if (wells_limit_lds(a.nwells, fp64) + win_lds > c->max_lds)
         return fail(c, OKA_ERR_ARG, "too many wells for LDS (%d)", a.nwells);
     int kind = kBmLdsFlat;
-    int blocks = nreal;
-    if (rasterize) {
+    if (rasterize)
         TRY(choose_bitmap(c, o, base_lds, a, &kind));
-        if (kind != kBmLdsFlat) {
-            // per-workgroup HBM regions: bound the resident set to what the
-            // LDS lets run at once
-            const size_t lds = base_lds + (kind == kBmTiled
-                                               ? (size_t)tile_lds_words(a.ntiles, a.tile_slots) * 4
-                                               : 0);
-            const int per_cu = (int)std::max<size_t>(1, std::min<size_t>(8, c->lds_per_cu / lds));
-            blocks = std::min(nreal, c->num_cu * per_cu);
-            const size_t words = kind == kBmTiled ? (size_t)a.ntiles * 32 : (size_t)a.nwords;
-            TRY(ensure(c, kSlotBitmap, sizeof(uint32_t) * words * blocks, &o2));
-            a.gbitmap = (uint32_t *)o2;
-            if (kind == kBmTiled)   // overflow tiles start empty; each flush leaves them so
-                TRY(fill_u32(c, a.gbitmap, (int64_t)words * blocks));
+    const size_t words = kind == kBmTiled ? (size_t)a.ntiles * 32 : (size_t)a.nwords;
+    const size_t lds = base_lds +
+                       (kind == kBmTiled     ? (size_t)tile_lds_words(a.ntiles, a.tile_slots) * 4
+                        : kind == kBmLdsFlat ? words * 4
+                                             : 0);
+    const int per_cu =
+        (int)std::max<size_t>(1, std::min<size_t>(8, c->lds_per_cu / std::max<size_t>(lds, 1)));
+    const int resident = c->num_cu * per_cu;   // or more than the registers let run
+    int blocks = kind == kBmLdsFlat ? nreal : std::min(nreal, resident);
+    // Realizations are taken from a queue where a workgroup has several, and
+    // the last ones shared (next_realization) where their particles outnumber
+    // a workgroup's lanes; few realizations then get workgroups for all their
+    // particles.  The window marks belong to one workgroup, and without the
+    // memory for the merged bitmaps nothing is shared.
+    const int nshared = std::min(nreal, resident);
+    const int spread = (int)std::min<int64_t>(
+        resident, (int64_t)nreal * ((o->npaths - 1) / kTraceBlock + 1));
+    bool refills = !marks && o->npaths > kTraceBlock &&
+                   (int64_t)(words * 4) * (nshared + std::max(nshared, spread)) <= kMaxShareBytes;
+    if (refills && words > 0) {
+        if (ensure(c, kSlotShareBits, sizeof(uint32_t) * words * nshared, &o2) == OKA_OK) {
+            a.share_bits = (uint32_t *)o2;
+            TRY(fill_u32(c, a.share_bits, (int64_t)words * nshared));
+        } else {
+            (void)hipGetLastError();
+            refills = false;
         }
+    }
+    if (!marks && (refills || nreal > blocks)) {
+        blocks = refills ? std::max(nshared, spread) : nshared;
+        a.share_first = refills ? nreal - nshared : nreal;
+        a.share_words = (int32_t)words;
+        const size_t counters = 1 + (size_t)(nreal - a.share_first);
+        TRY(ensure(c, kSlotShare, sizeof(int32_t) * counters, &o2));
+        a.share = (int32_t *)o2;
+        TRY(fill_u32(c, a.share, (int64_t)counters));
+    }
+    if (kind != kBmLdsFlat) {
+        // per-workgroup HBM regions, of the workgroups that the LDS lets run at once
+        TRY(ensure(c, kSlotBitmap, sizeof(uint32_t) * words * blocks, &o2));
+        a.gbitmap = (uint32_t *)o2;
+        if (kind == kBmTiled)   // overflow tiles start empty; each flush leaves them so
+            TRY(fill_u32(c, a.gbitmap, (int64_t)words * blocks));
     }
     if (!fp64) {   // grown in steps of 8,192 wells
         TRY(ensure(c, kSlotWells32, sizeof(float2) * ((a.nwells + 8191) / 8192 * 8192), &o2));

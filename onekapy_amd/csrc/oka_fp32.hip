@@ -1,6 +1,6 @@
 // oka_fp32.hip -- FP32 particle tracing for gfx950 (confined or unconfined
-// velocity): one 256-lane workgroup per realization, grid-stride over
-// realizations.  The step,
+// velocity): one workgroup of up to 256 lanes per realization, taken
+// from a queue, the last ones shared (next_realization).  The step,
 // field and rasterizer are in oka_fp32_dev.h.  Results are not bit-identical
 // to the FP64 path; the difference in capture probability is reported against
 // the FP64-exact mode.
@@ -30,6 +30,7 @@ k_trace_fp32(TraceArgs a)
     uint32_t *s_bm = reinterpret_cast<uint32_t *>(smem4 + (kConfined ? 1 : 2) * nw4);
     using Bits = typename std::conditional<kKind == kBmTiled, TileBits, FlatBits>::type;
     __shared__ int s_next;
+    __shared__ ShareLds s_share;
     __shared__ unsigned long long s_stat[kStatCount];
     __shared__ float s_reg[11];
 
@@ -67,7 +68,9 @@ k_trace_fp32(TraceArgs a)
             s_win[c] = 0u;
     }
 
-    for (int r = blockIdx.x; r < a.nreal; r += gridDim.x) {
+    for (int r = next_realization(a, -1, s_share); r < a.nreal;
+         r = next_realization(a, r, s_share)) {
+        int32_t *const shared = shared_counter(a, r);
         if (tid < kStatCount)
             s_stat[tid] = 0;
         const double bn = a.b[r] * a.n[r];
@@ -121,7 +124,7 @@ k_trace_fp32(TraceArgs a)
 
         Trace32 s;
         Epoch32 ep;
-        int p = tid;
+        int p = shared ? claim_one(shared) : tid;
         bool have = p < P;
         bool live = false, fresh = false;
         bool a_done = false;   // the disk around the trace's current point is marked
@@ -189,16 +192,17 @@ k_trace_fp32(TraceArgs a)
                     a.trace_status[k] = s.status;
                 if (a.trace_steps)
                     a.trace_steps[k] = s.att;
-                p = atomicAdd(&s_next, 1);
+                p = shared ? claim_one(shared) : atomicAdd(&s_next, 1);
                 have = p < P;
             }
         }
         __syncthreads();
         if (a.rasterize) {
+            uint32_t *const merged = merged_bits(a, r, traced(s_stat));
             if constexpr (kKind == kBmTiled)
-                atomicAdd(&s_stat[kStatVisited], flush_tiles(a, bits, s_win));
+                atomicAdd(&s_stat[kStatVisited], flush_tiles(a, bits, s_win, merged));
             else
-                atomicAdd(&s_stat[kStatVisited], flush_bitmap(a, bits.bm, s_win));
+                atomicAdd(&s_stat[kStatVisited], flush_bitmap(a, bits.bm, s_win, merged));
         }
         __syncthreads();
         if (s_win) {

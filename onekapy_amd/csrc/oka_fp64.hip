@@ -9,7 +9,7 @@
 //   Dormand-Prince     oneka/capturezone.py:198-253
 //   segment raster     oneka/probabilityfield.py:292-310, 407-427
 //
-// Work layout: one workgroup per realization (grid-stride over realizations),
+// Work layout: one workgroup per realization (taken from a queue, the last ones shared),
 // one particle per lane with lanes refilled from an LDS counter as their traces
 // end, the realization's discharges staged in LDS, and the realization's visited-node
 // bitmap in LDS (or HBM for grids too large for it).  At the end of the
@@ -45,9 +45,9 @@ struct Chron<kModeLdsBitmap> {
         for (int w = threadIdx.x; w < a.nwords; w += blockDim.x)
             bits.bm[w] = 0u;
     }
-    __device__ unsigned long long flush(const TraceArgs &a, unsigned int *s_win)
+    __device__ unsigned long long flush(const TraceArgs &a, unsigned int *s_win, uint32_t *merged)
     {
-        return flush_bitmap(a, bits.bm, s_win);
+        return flush_bitmap(a, bits.bm, s_win, merged);
     }
 };
 
@@ -58,9 +58,9 @@ template <>
 struct Chron<kModeTiledBitmap> {
     TileBits bits;
     __device__ void begin(const TraceArgs &) {}
-    __device__ unsigned long long flush(const TraceArgs &a, unsigned int *s_win)
+    __device__ unsigned long long flush(const TraceArgs &a, unsigned int *s_win, uint32_t *merged)
     {
-        return flush_tiles(a, bits, s_win);
+        return flush_tiles(a, bits, s_win, merged);
     }
 };
 
@@ -68,11 +68,12 @@ template <>
 struct Chron<kModeVertices> {
     FlatBits bits;   // unused
     __device__ void begin(const TraceArgs &) {}
-    __device__ unsigned long long flush(const TraceArgs &, unsigned int *) { return 0; }
+    __device__ unsigned long long flush(const TraceArgs &, unsigned int *, uint32_t *) { return 0; }
 };
 
-// One workgroup per realization (grid-stride), one trace per lane, lanes
-// refilled from the LDS counter s_next when their trace ends.
+// One workgroup per realization (next_realization), one trace per lane, lanes
+// refilled from the LDS counter s_next, or the shared counter of one of the last
+// realizations, when their trace ends.
 // Both tracers are held to 128 VGPRs (4 waves per SIMD).  The confined one
 // spills one 64-bit value, stored before the realization loop and read after
 // it, and is 3 % faster than with the 150 the compiler picks.  The unconfined
@@ -87,6 +88,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
     extern __shared__ double smem[];
     double *s_nq = smem;   // the realization's -q
     __shared__ int s_next;
+    __shared__ ShareLds s_share;
     __shared__ unsigned long long s_stat[kStatCount];
 
     const int tid = threadIdx.x;
@@ -111,7 +113,9 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
         for (int c = threadIdx.x; c < a.w_nr * a.w_nc; c += blockDim.x)
             s_win[c] = 0u;
 
-    for (int r = blockIdx.x; r < a.nreal; r += gridDim.x) {
+    for (int r = next_realization(a, -1, s_share); r < a.nreal;
+         r = next_realization(a, r, s_share)) {
+        int32_t *const shared = shared_counter(a, r);
         if (tid < kStatCount)
             s_stat[tid] = 0;
         int ok = min(plain_origin(a.xo), plain_origin(a.yo));
@@ -137,7 +141,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
 
         Trace64 s;
         EpochReg ep;
-        int p = tid;
+        int p = shared ? claim_one(shared) : tid;
         bool have = p < P;
         bool live = false, fresh = false;
         for (;;) {
@@ -188,7 +192,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
                     a.trace_steps[k] = s.att;
                 if (kVerts)
                     a.nverts[k] = s.acc + 1;
-                p = atomicAdd(&s_next, 1);
+                p = shared ? claim_one(shared) : atomicAdd(&s_next, 1);
                 have = p < P;
             }
         }
@@ -202,7 +206,7 @@ __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)
         __syncthreads();
 
         if (raster)
-            atomicAdd(&s_stat[kStatVisited], ch.flush(a, s_win));
+            atomicAdd(&s_stat[kStatVisited], ch.flush(a, s_win, merged_bits(a, r, traced(s_stat))));
         __syncthreads();
         if (s_win) {
             store_window(a, r, s_win);

@@ -3,7 +3,8 @@ particles are given, the counts, per-trace statuses and statistics are those of
 the pool, which deals out particles on its own."""
 import pytest
 
-from onekapy_amd import _lib, sites
+from onekapy_amd import _lib
+from onekapy_amd.sites import fixed_field
 from helpers import oracle_fit_draw, small_site
 from test_gpu_pool import _both
 
@@ -19,3 +20,18 @@ def test_lanes_for_the_particles(gpu_ctx, npaths, precision):
     _, _, coef = oracle_fit_draw(s, d)
     print(f"npaths {npaths} precision {precision}", flush=True)
     _both(s, d, coef, s.fixed_field(), s.umbra, precision)
+
+
+# (realizations, particles, field spacing): one realization spread over many
+# workgroups; fewer realizations than CUs; every workgroup's last one shared;
+# the fine lattices' bitmaps are tiled
+@pytest.mark.parametrize("nreal,npaths,spacing", [
+    (1, 257, None), (1, 3000, None), (3, 1000, None), (700, 320, None), (2500, 300, None),
+    (2, 1500, 5.0), (600, 20, 5.0)])
+@pytest.mark.parametrize("precision", [_lib.FP64_EXACT, _lib.FP32], ids=["fp64", "fp32"])
+def test_shared_realizations(gpu_ctx, nreal, npaths, spacing, precision):
+    s, d = small_site(nreal=nreal, npaths=npaths)
+    _, _, coef = oracle_fit_draw(s, d)
+    pf = s.fixed_field() if spacing is None else fixed_field(s.xt, s.yt, spacing, 900, 950)
+    print(f"{nreal} x {npaths} spacing {spacing} precision {precision}", flush=True)
+    _both(s, d, coef, pf, s.umbra, precision)

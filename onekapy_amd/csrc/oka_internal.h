@@ -109,40 +109,64 @@ struct TraceArgs {
     const int32_t *far_wbox;        // [nwells][2]: each well's box column and row
 };
 
-// One marked node of a realization: its count (probabilityfield.py:357-359)
-// and, when a window is requested, its cell's LDS word: the count of the
-// cell's marked nodes, or with node masks (cells of at most 4 x 4 nodes) the
-// bit (row in cell) * cell + (column in cell).
-__device__ inline void count_node(const TraceArgs &a, int row, int col, unsigned int *s_win)
+// The window cell of a marked node: its LDS word takes the count of the cell's
+// marked nodes, or with node masks (cells of at most 4 x 4 nodes) the bit
+// (row in cell) * cell + (column in cell).
+__device__ inline void window_node(const TraceArgs &a, int row, int col, unsigned int *s_win)
 {
-    if (a.counts)
-        atomicAdd(&a.counts[(int64_t)row * a.gncols + col], 1);
-    if (s_win) {
-        const int ci = row - a.w_row0, cj = col - a.w_col0;
-        if (ci >= 0 && cj >= 0) {
-            const int r = ci / a.w_cell, c = cj / a.w_cell;
-            if (r < a.w_nr && c < a.w_nc) {
-                if (a.wmasks)
-                    atomicOr(&s_win[r * a.w_nc + c],
-                             1u << ((ci - r * a.w_cell) * a.w_cell + (cj - c * a.w_cell)));
-                else
-                    atomicAdd(&s_win[r * a.w_nc + c], 1u);
-            }
+    const int ci = row - a.w_row0, cj = col - a.w_col0;
+    if (ci >= 0 && cj >= 0) {
+        const int r = ci / a.w_cell, c = cj / a.w_cell;
+        if (r < a.w_nr && c < a.w_nc) {
+            if (a.wmasks)
+                atomicOr(&s_win[r * a.w_nc + c],
+                         1u << ((ci - r * a.w_cell) * a.w_cell + (cj - c * a.w_cell)));
+            else
+                atomicAdd(&s_win[r * a.w_nc + c], 1u);
         }
     }
 }
 
-// The nodes of one tile row: bit b of `bits` is column col0 + b of `row`.
-__device__ inline unsigned long long count_bits(const TraceArgs &a, int row, int col0,
-                                                uint32_t bits, unsigned int *s_win)
+// The marked nodes of a realization (probabilityfield.py:357-359) in the words
+// of one wave: lane l brings `bits`, whose bit b is the node of flat index
+// first + b.  Every lane of the wave calls it.  The words are taken two at a
+// time, a bit per lane, so that each atomic instruction adds to two runs of
+// neighbouring counts: with a word per lane every lane of it fell into a cache
+// line of its own, and the counts' L2 traffic bound short traces on fine grids
+// (8,000 realizations x 100 particles, FP32, 5 years, 1600 x 1600 nodes of 5 m:
+// 10.1 ms, now 6.5).
+// Returns the lane's number of nodes.
+__device__ inline unsigned long long count_words(const TraceArgs &a, uint32_t bits, int first,
+                                                 unsigned int *s_win)
 {
-    const unsigned long long n = (unsigned long long)__popc(bits);
-    while (bits) {
-        const int col = col0 + __ffs(bits) - 1;
-        bits &= bits - 1u;
-        count_node(a, row, col, s_win);
+    const int lane = threadIdx.x & 63, b = lane & 31;
+    unsigned long long todo = __ballot(bits != 0u);
+    while (todo) {
+        const int j0 = __ffsll(todo) - 1;
+        todo &= todo - 1;
+        const int j1 = todo ? __ffsll(todo) - 1 : j0;
+        uint32_t w1 = todo ? __builtin_amdgcn_readlane(bits, j1) : 0u;
+        todo &= todo - 1;
+        const uint32_t w0 = __builtin_amdgcn_readlane(bits, j0);
+        const int f0 = __builtin_amdgcn_readlane(first, j0);
+        const int f1 = __builtin_amdgcn_readlane(first, j1);
+        if (((lane < 32 ? w0 : w1) >> b) & 1u) {
+            const int idx = (lane < 32 ? f0 : f1) + b;
+            if (a.counts)
+                atomicAdd(&a.counts[idx], 1);
+            if (s_win) {
+                const int row = idx / a.gncols;
+                window_node(a, row, idx - row * a.gncols, s_win);
+            }
+        }
     }
-    return n;
+    return (unsigned long long)__popc(bits);
+}
+
+// The flat index of the first node of word `row` of tile t.
+__device__ __forceinline__ int tile_first(const TraceArgs &a, int t, int row)
+{
+    return ((t / a.tiles_x) * 32 + row) * a.gncols + (t % a.tiles_x) * 32;
 }
 
 // n consecutive bits starting at bit b of a word (1 <= n <= 32 - b; for
@@ -400,15 +424,11 @@ __device__ inline unsigned long long flush_bitmap(const TraceArgs &a, const uint
                                                   unsigned int *s_win, uint32_t *merged)
 {
     unsigned long long vis = 0;
-    for (int w = threadIdx.x; w < a.nwords; w += blockDim.x) {
-        uint32_t bits = merge_word(merged, w, bm[w]);
-        vis += (unsigned long long)__popc(bits);
-        while (bits) {
-            const int idx = w * 32 + __ffs(bits) - 1;
-            bits &= bits - 1u;
-            const int row = idx / a.gncols;
-            count_node(a, row, idx - row * a.gncols, s_win);
-        }
+    const int lane = threadIdx.x & 63;
+    for (int w0 = threadIdx.x - lane; w0 < a.nwords; w0 += blockDim.x) {
+        const int w = w0 + lane;
+        const uint32_t bits = w < a.nwords ? merge_word(merged, w, bm[w]) : 0u;
+        vis += count_words(a, bits, w * 32, s_win);
     }
     return vis;
 }
@@ -421,27 +441,29 @@ __device__ inline unsigned long long flush_tiles(const TraceArgs &a, TileBits &t
     unsigned long long vis = 0;
     const int handed = *tb.nslots;
     const int ns = handed < tb.maxslots ? handed : tb.maxslots;
-    for (int w = threadIdx.x; w < ns * 32; w += blockDim.x) {
-        const int t = tb.slot_tile[w >> 5];
-        uint32_t bits = tb.slots[w];
-        if (t < 0 || !bits)
-            continue;
-        tb.slots[w] = 0u;
-        bits = merge_word(merged, (int64_t)t * 32 + (w & 31), bits);
-        vis += count_bits(a, (t / tb.tiles_x) * 32 + (w & 31), (t % tb.tiles_x) * 32, bits, s_win);
+    const int lane = threadIdx.x & 63;
+    for (int w0 = threadIdx.x - lane; w0 < ns * 32; w0 += blockDim.x) {
+        const int w = w0 + lane;   // 32 words a slot: whole waves or halves of them
+        const int t = w < ns * 32 ? tb.slot_tile[w >> 5] : -1;
+        uint32_t bits = t < 0 ? 0u : tb.slots[w];
+        if (bits) {
+            tb.slots[w] = 0u;
+            bits = merge_word(merged, (int64_t)t * 32 + (w & 31), bits);
+        }
+        vis += count_words(a, bits, t < 0 ? 0 : tile_first(a, t, w & 31), s_win);
     }
     if (handed > tb.maxslots) {   // some tiles went to HBM
-        for (int w = threadIdx.x; w < tb.ntiles * 32; w += blockDim.x) {
-            const int t = w >> 5;
-            if (tb.tmap[t] != kTileOverflow)
-                continue;
-            uint32_t bits = tb.hbm[w];
-            if (!bits)
-                continue;
-            tb.hbm[w] = 0u;
-            bits = merge_word(merged, w, bits);
-            vis += count_bits(a, (t / tb.tiles_x) * 32 + (w & 31), (t % tb.tiles_x) * 32, bits,
-                              s_win);
+        for (int w0 = threadIdx.x - lane; w0 < tb.ntiles * 32; w0 += blockDim.x) {
+            const int w = w0 + lane, t = w >> 5;
+            uint32_t bits = 0u;
+            if (t < tb.ntiles && tb.tmap[t] == kTileOverflow) {
+                bits = tb.hbm[w];
+                if (bits) {
+                    tb.hbm[w] = 0u;
+                    bits = merge_word(merged, w, bits);
+                }
+            }
+            vis += count_words(a, bits, tile_first(a, t, w & 31), s_win);
         }
     }
     __syncthreads();

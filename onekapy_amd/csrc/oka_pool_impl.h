@@ -396,28 +396,29 @@ __device__ void flush_slot(const PoolArgs &P, const PoolLds<Prec> &L, int s)
     const PoolBits b = slot_bits(P, L, s, A.tiles_x);
     unsigned long long vis = 0;
     if (A.rasterize) {
+        static_assert(kHash * 32 % kWave == 0, "every lane calls count_words");
         for (int k = threadIdx.x; k < kHash * 32; k += kWave) {
             const uint32_t e = b.keys[k >> 5];
-            if (e == kKeyEmpty)
-                continue;
-            const uint32_t t = e >> kValBits;
-            uint32_t *w = b.tile_words(t, e & kValMask) + (k & 31);
-            const uint32_t bits = *w;
-            if (!bits)
-                continue;
-            *w = 0u;
-            vis += count_bits(A, (int)(t / A.tiles_x) * 32 + (k & 31), (int)(t % A.tiles_x) * 32,
-                              bits, nullptr);
+            const int t = (int)(e >> kValBits);
+            uint32_t bits = 0u;
+            if (e != kKeyEmpty) {
+                uint32_t *w = b.tile_words(t, e & kValMask) + (k & 31);
+                bits = *w;
+                if (bits)
+                    *w = 0u;
+            }
+            vis += count_words(A, bits, bits ? tile_first(A, t, k & 31) : 0, nullptr);
         }
         if (h.hash_full) {   // unmapped tiles: scan the whole HBM region
-            for (int k = threadIdx.x; k < A.ntiles * 32; k += kWave) {
-                const uint32_t bits = b.hbm[k];
-                if (!bits)
-                    continue;
-                b.hbm[k] = 0u;
-                const int t = k >> 5;
-                vis += count_bits(A, (t / A.tiles_x) * 32 + (k & 31), (t % A.tiles_x) * 32, bits,
-                                  nullptr);
+            for (int k0 = 0; k0 < A.ntiles * 32; k0 += kWave) {
+                const int k = k0 + (int)threadIdx.x;
+                uint32_t bits = 0u;
+                if (k < A.ntiles * 32) {
+                    bits = b.hbm[k];
+                    if (bits)
+                        b.hbm[k] = 0u;
+                }
+                vis += count_words(A, bits, tile_first(A, k >> 5, k & 31), nullptr);
             }
         }
     }
@@ -506,25 +507,44 @@ __device__ void merge_slot(const PoolArgs &P, const PoolLds<Prec> &L, int s)
         unsigned long long vis = 0;
         if (A.rasterize) {
             const int dwords = (A.ntiles + 31) / 32;
-            for (int dw = 0; dw < dwords; ++dw) {
-                uint32_t dbits = __hip_atomic_load(&rd[dw], __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-                while (dbits) {
-                    const int t = dw * 32 + __ffs(dbits) - 1;
-                    dbits &= dbits - 1u;
-                    if (threadIdx.x < 32) {
-                        uint32_t *w = &rb[(int64_t)t * 32 + threadIdx.x];
-                        const uint32_t bits = __hip_atomic_load(w, __ATOMIC_RELAXED,
-                                                                __HIP_MEMORY_SCOPE_AGENT);
-                        if (bits) {
-                            __hip_atomic_store(w, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            vis += count_bits(A, (t / A.tiles_x) * 32 + (int)threadIdx.x,
-                                              (t % A.tiles_x) * 32, bits, nullptr);
+            for (int d0 = 0; d0 < dwords; d0 += kWave) {
+                const int dl = d0 + (int)threadIdx.x;
+                const uint32_t dirty = dl < dwords
+                                           ? __hip_atomic_load(&rd[dl], __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_AGENT)
+                                           : 0u;
+                if (dirty)
+                    __hip_atomic_store(&rd[dl], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (unsigned long long m = __ballot(dirty != 0u); m; m &= m - 1) {
+                    const int dw = d0 + __ffsll(m) - 1;
+                    uint32_t dbits = __builtin_amdgcn_readlane(dirty, __ffsll(m) - 1);
+                    while (dbits) {   // up to 8 tiles at a time, their words in flight together
+                        constexpr int kPairs = 4;
+                        uint32_t bits[kPairs];
+                        int t[kPairs];
+#pragma unroll
+                        for (int i = 0; i < kPairs; ++i) {
+                            const int t0 = dbits ? __ffs(dbits) - 1 : -1;
+                            dbits &= dbits - 1u;
+                            const int t1 = dbits ? __ffs(dbits) - 1 : -1;
+                            dbits &= dbits - 1u;
+                            const int tb = threadIdx.x < 32 ? t0 : t1;
+                            t[i] = dw * 32 + tb;
+                            bits[i] = tb < 0 ? 0u
+                                             : __hip_atomic_load(
+                                                   &rb[(int64_t)t[i] * 32 + (threadIdx.x & 31)],
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        }
+#pragma unroll
+                        for (int i = 0; i < kPairs; ++i) {
+                            if (bits[i])
+                                __hip_atomic_store(&rb[(int64_t)t[i] * 32 + (threadIdx.x & 31)], 0u,
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            vis += count_words(A, bits[i], tile_first(A, t[i], threadIdx.x & 31),
+                                               nullptr);
                         }
                     }
                 }
-                if (threadIdx.x == 0)
-                    __hip_atomic_store(&rd[dw], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         for (int off = 32; off > 0; off >>= 1)

@@ -929,9 +929,20 @@ int choose_bitmap(oka_ctx *c, const oka_trace_opts *o, size_t base_lds, TraceArg
     const bool flat_fits = base_lds + (size_t)a.nwords * 4 <= budget;
     a.tiles_x = (a.gncols + 31) / 32;
     const int64_t ntiles = (int64_t)a.tiles_x * ((a.gnrows + 31) / 32);
+    const size_t fixed = base_lds + (size_t)(ntiles + 1) * 4;
     int64_t slots = 0;
-    if (base_lds + (size_t)(ntiles + 1) * 4 < budget)
-        slots = (int64_t)(budget - base_lds - (size_t)(ntiles + 1) * 4) / (4 * 33);
+    // the LDS share of the most workgroups per CU that leaves enough slots (the
+    // whole budget for a caller's own number of them)
+    const int waves = trace_block(o->npaths) / 64;
+    for (int per_cu = o->tile_slots > 0 ? 2 : waves <= 2 ? 8 : 4; slots < kEnoughTileSlots;
+         --per_cu) {
+        const size_t share = per_cu < 3 ? budget
+                                        : std::min(budget, c->lds_per_cu / per_cu / kLdsGrain *
+                                                               kLdsGrain - kLdsOwn);
+        slots = fixed < share ? (int64_t)(share - fixed) / (4 * 33) : 0;
+        if (per_cu < 3)
+            break;
+    }
     if (o->tile_slots > 0)
         slots = std::min<int64_t>(slots, o->tile_slots);
     a.ntiles = (int32_t)ntiles;

@@ -27,6 +27,16 @@ constexpr int kLdsBudget = 57344;           // LDS bytes per trace workgroup (2 
 enum BitmapKind { kBmLdsFlat = 0, kBmTiled = 1, kBmHbmFlat = 2 };
 constexpr int kTileEmpty = -1, kTileOverflow = -2;
 constexpr int kMinTileSlots = 16;
+// Tile slots from which on more workgroups per CU are worth more than more
+// slots.  25 wells, 2 workgroups a CU (56 KiB each) -> the rule: 1600 x 1600 nodes,
+// 1,000 realizations x 1,000 particles (4 a CU, 229 slots) FP64 19.5 -> 17.7 ms, FP32
+// 8.2 -> 6.1; 4,000 x 100 (6 a CU, 122 slots) 21.7 -> 13.2 and 8.4 -> 5.0;
+// 8,000 x 30 36.0 -> 16.8 and 14.7 -> 7.0; 3000 x 3000, 1,000 x 1,000 (3 a CU, 132
+// slots) 34.6 -> 31.3 and 14.7 -> 11.9.  Below, tiles overflow into HBM: 3400 x
+// 3400 FP32 with 60 slots at 3 a CU 21.5 ms against 14.7 with 85 at 2.
+constexpr int kEnoughTileSlots = 96;
+constexpr size_t kLdsGrain = 2048;          // LDS is given out in steps no larger than this
+constexpr size_t kLdsOwn = 256;             // the trace kernels' own LDS variables, at most
 
 // Far-well expansions of the FP32 pool (fp32::FarField): the number of
 // coefficients each box keeps and evaluates (those above a plan's order are

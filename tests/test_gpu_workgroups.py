@@ -35,3 +35,15 @@ def test_shared_realizations(gpu_ctx, nreal, npaths, spacing, precision):
     pf = s.fixed_field() if spacing is None else fixed_field(s.xt, s.yt, spacing, 900, 950)
     print(f"{nreal} x {npaths} spacing {spacing} precision {precision}", flush=True)
     _both(s, d, coef, pf, s.umbra, precision)
+
+
+# lattices (nodes a side) whose tile index leaves 8, 4 and 3 workgroups' LDS
+# enough slots, that of 2 only, and hardly any
+@pytest.mark.parametrize("nside,npaths", [(700, 40), (1500, 40), (1500, 300), (2900, 200),
+                                          (3300, 70), (3550, 30)])
+def test_tiles_for_the_workgroups(gpu_ctx, nside, npaths):
+    s, d = small_site(nreal=5, npaths=npaths)
+    _, _, coef = oracle_fit_draw(s, d)
+    pf = fixed_field(s.xt, s.yt, 6000.0 / nside, nside, nside)
+    print(f"nside {nside} npaths {npaths}", flush=True)
+    _both(s, d, coef, pf, s.umbra, _lib.FP64_EXACT)

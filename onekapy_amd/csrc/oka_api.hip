@@ -1100,9 +1100,9 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
     // a workgroup's lanes; few realizations then get workgroups for all their
     // particles.  The window marks belong to one workgroup, and without the
     // memory for the merged bitmaps nothing is shared.
-    const int nshared = std::min(nreal, resident);
+    const int nshared = std::min(nreal, std::min(resident, 5 * c->num_cu));   // 4 or 5 run at once
     const int spread = (int)std::min<int64_t>(
-        resident, (int64_t)nreal * ((o->npaths - 1) / kTraceBlock + 1));
+        c->num_cu, (int64_t)nreal * ((o->npaths - 1) / kTraceBlock + 1));
     bool refills = !marks && o->npaths > kTraceBlock &&
                    (int64_t)(words * 4) * (nshared + std::max(nshared, spread)) <= kMaxShareBytes;
     if (refills && words > 0) {
@@ -1115,10 +1115,10 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
         }
     }
     if (!marks && (refills || nreal > blocks)) {
-        blocks = refills ? std::max(nshared, spread) : nshared;
+        blocks = refills ? std::max(nshared, spread) : std::min(nreal, resident);
         a.share_first = refills ? nreal - nshared : nreal;
         a.share_words = (int32_t)words;
-        const size_t counters = 1 + (size_t)(nreal - a.share_first);
+        const size_t counters = kShareStride * (1 + (size_t)(nreal - a.share_first));
         TRY(ensure(c, kSlotShare, sizeof(int32_t) * counters, &o2));
         a.share = (int32_t *)o2;
         TRY(fill_u32(c, a.share, (int64_t)counters));

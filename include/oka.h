@@ -155,8 +155,9 @@ typedef struct {
                                 where the plan pays; < 0: every well summed directly */
 } oka_trace_opts;
 
-/* How particles are scheduled on the GPU.  WORKGROUP: one 256-lane workgroup
- * per realization, its lanes refilled with the realization's particles.
+/* How particles are scheduled on the GPU.  WORKGROUP: one workgroup of
+ * up to 256 lanes per realization, its lanes refilled with the realization's
+ * particles; workgroups that run out of realizations help with the last ones.
  * POOL (no window marks): a persistent grid of single waves
  * working through a queue shared by all waves of chunks of pool_chunk
  * particles; each wave keeps pool_slots chunks in flight and refills a lane
@@ -508,8 +509,8 @@ int oka_field_smooth(oka_ctx *ctx, int32_t nrows, int32_t ncols, const double *p
                      uint32_t flags);
 
 /* The impact curve's probabilities (visualize.py:382): pr = the n values of
- * pgrid / total_weight sorted in descending order (a radix sort on the device;
- * for fields of whole counts oka_count_histogram gives the same array).
+ * pgrid / total_weight sorted in descending order (on the device: counted
+ * for fields of whole counts, except in asynchronous calls, else a radix sort).
  * pgrid and pr follow flags. */
 int oka_field_sorted_probabilities(oka_ctx *ctx, int64_t n, const double *pgrid,
                                    double total_weight, double *pr, uint32_t flags);

@@ -115,6 +115,38 @@ def test_training_step_gradient_matches_oracle(gpu_ctx, nh, nout, B):
         assert rel < 2e-2, (name, rel)
 
 
+@pytest.mark.parametrize("nin,nh,nout,B", [(13, 64, 64, 64), (34, 128, 192, 128)])
+def test_adam_rounds_as_written(gpu_ctx, nin, nh, nout, B):
+    """Three Adam steps, each from the gradient call's own gradient (at these
+    batches the step splits no dW, so it is the step's too): the parameters are
+    bit for bit those of m = fma(g, 1 - b1, b1 m), v = fma(b2, v, (1 - b2) g g)
+    and p - lr (m c1) / (sqrt(v c2) + eps) in float."""
+    f32, b1, b2, eps, lr = np.float32, np.float32(0.9), np.float32(0.999), np.float32(1e-8), \
+        np.float32(0.25)
+    one = f32(1)
+
+    def fma(a, b, c):   # float products are exact in 64 bits of mantissa
+        return (np.longdouble(a) * np.longdouble(b) + np.longdouble(c)).astype(f32)
+
+    net = SurrogateMLP(nin, nh, nout, max_batch=B, seed=31)
+    rng = np.random.default_rng(32)
+    p = net.get_params()
+    m, v = np.zeros_like(p), np.zeros_like(p)
+    order = np.arange(B, dtype=np.int32)
+    for t in (1, 2, 3):
+        x = rng.normal(0, 1, (B, nin)).astype(f32)
+        marks = rng.integers(0, 26, (B, nout)).astype(np.uint8)
+        g, _ = net.grad(x, marks, 1.0 / 25.0)
+        net.ctx.check(net.ctx.lib.oka_mlp_train(
+            net.h, B, x.ctypes.data, marks.ctypes.data, 1.0 / 25.0, order.ctypes.data, B, 1, lr,
+            b1, b2, eps, None, 0))
+        m = fma(g, one - b1, b1 * m)
+        v = fma(b2, v, (one - b2) * g * g)
+        c1, c2 = (f32(1.0 / (1.0 - np.exp(t * np.log(np.float64(b))))) for b in (b1, b2))
+        p = p - lr * (m * c1) / (np.sqrt(v * c2) + eps)
+        assert np.array_equal(net.get_params(), p), t
+
+
 def test_training_fits_a_smooth_target(gpu_ctx):
     rng = np.random.default_rng(5)
     nin, nout = 34, 256

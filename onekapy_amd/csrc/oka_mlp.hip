@@ -725,8 +725,9 @@ using namespace mlp;
 // layers of 8,192 rows: 256 big tiles, 16 us; 1,024 small ones, 9 us).  A dW
 // product beside its dX takes them from one workgroup per CU on: its K is
 // long, and split plans raise the count (dW3 with dX3 at batch 2,048: 32 us
-// big, 47 small).
-static bool use_big_tiles(const GemmArgs &g1, const GemmArgs *g2)
+// big, 47 small).  So does the loss product, whose epilogue writes both copies
+// of its gradient (batch 1,024, 256 big tiles: 20.4 us big, 24.3 small).
+static bool use_big_tiles(int e1, const GemmArgs &g1, const GemmArgs *g2)
 {
     // compute units of the current device (the caller has set it)
     int dev = 0, num_cu = 0;
@@ -737,12 +738,13 @@ static bool use_big_tiles(const GemmArgs &g1, const GemmArgs *g2)
     auto fits = [](const GemmArgs &g) { return g.M % 128 == 0 && g.N % 128 == 0; };
     if (!fits(g1) || (g2 && !fits(*g2)))
         return false;
-    return gemm_tiles(g1, 1) + (g2 ? gemm_tiles(*g2, 1) : 0) >= (g2 ? 1 : 2) * num_cu;
+    return gemm_tiles(g1, 1) + (g2 ? gemm_tiles(*g2, 1) : 0) >=
+           (g2 || e1 == kEpiLossGrad ? 1 : 2) * num_cu;
 }
 
 int gemm2_workgroups(const GemmArgs &g1, const GemmArgs *g2)
 {
-    const bool big = use_big_tiles(g1, g2);
+    const bool big = use_big_tiles(kEpiPartialF32, g1, g2);
     return gemm_tiles(g1, big) + (g2 ? gemm_tiles(*g2, big) : 0);
 }
 
@@ -753,7 +755,7 @@ hipError_t launch_gemm2(int e1, const GemmArgs &g1, int e2, const GemmArgs &g2, 
     if (e2 != kEpiNone && (g2.M % kTile || g2.N % kTile || g2.splits < 1 ||
                            g2.K % (g2.splits * kBK)))
         return hipErrorInvalidValue;
-    const bool big = use_big_tiles(g1, e2 == kEpiNone ? nullptr : &g2);
+    const bool big = use_big_tiles(e1, g1, e2 == kEpiNone ? nullptr : &g2);
     if (e1 == kEpiAccum && e2 == kEpiNone) {
         // 4 row tiles a workgroup: 2 workgroups per CU at 8,192 rows of 4,096
         // outputs (66 us; 86 with 8 row tiles, one workgroup per CU)

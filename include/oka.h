@@ -89,7 +89,17 @@ int oka_ctx_device_info(oka_ctx *ctx, oka_device_info *out);
 int oka_ctx_create(oka_ctx **out, int device);
 void oka_ctx_destroy(oka_ctx *ctx);
 const char *oka_last_error(const oka_ctx *ctx);
-/* Use the caller's HIP stream (a hipStream_t), or NULL for the library's own. */
+/* Use the caller's HIP stream (a hipStream_t), or NULL for the library's own.
+ * Nothing waits for what earlier calls left running (OKA_ASYNC) on the stream
+ * before.  Most calls keep scratch memory in the context: let those end, or
+ * have the new stream wait for them, before the next call, and capture none of
+ * them in a HIP graph.  The exception is oka_trace_chronicle with OKA_ASYNC |
+ * OKA_PTR_DEVICE, no stats, epochs (nepochs > 0), the workgroup schedule and a
+ * grid whose bitmap fits LDS.  Such calls may overlap one another on several
+ * streams.  A HIP graph may capture them, and stays good whatever the context
+ * does until oka_ctx_destroy.  While one of them runs, or under capture, a call
+ * does without the launch state that workgroups share (oka_trace_opts.schedule),
+ * so it takes longer. */
 int oka_ctx_set_stream(oka_ctx *ctx, void *hip_stream);
 void *oka_ctx_stream(oka_ctx *ctx);
 int oka_ctx_synchronize(oka_ctx *ctx);

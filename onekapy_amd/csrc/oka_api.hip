@@ -546,7 +546,8 @@ int oka_ctx_create(oka_ctx **out, int device)
     hipDeviceProp_t prop;
     if (hipSetDevice(device) != hipSuccess || hipGetDeviceProperties(&prop, device) != hipSuccess ||
         hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
+        hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
+        hipEventCreateWithFlags(&c->launch_done, hipEventDisableTiming) != hipSuccess) {
         delete c;
         return OKA_ERR_DEVICE;
     }
@@ -570,11 +571,14 @@ void oka_ctx_destroy(oka_ctx *c)
         return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    if (c->launch_busy)
+        (void)hipEventSynchronize(c->launch_done);
     for (auto &b : c->buf)
         if (b.p)
             (void)hipFree(b.p);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
+    if (c->launch_done) (void)hipEventDestroy(c->launch_done);
     if (c->own) (void)hipStreamDestroy(c->own);
     delete c;
 }
@@ -916,6 +920,31 @@ int run_pool(oka_ctx *c, const TraceArgs *sites, int nsites, const oka_trace_opt
     return OKA_OK;
 }
 
+// Whether this call may keep launch state in the context's slots (the queue,
+// the merged bitmaps, the FP32 wells' places): not while a launch on another
+// stream may still be using it, and not under capture, whose graph would hold
+// their addresses after they have grown.  Such a call launches a workgroup a
+// realization, with the wells' records in its LDS: 10^4 x 1000 particles of the
+// benchmark's 25-well site FP64 169.4 ms instead of 164.3, FP32 57.1 instead
+// of 51.1.
+bool launch_state_free(oka_ctx *c)
+{
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    if (capture != hipStreamCaptureStatusNone)
+        return false;
+    if (!c->launch_busy)
+        return true;
+    if (c->launch_stream == c->stream)   // in order, but for a new stream under an old handle
+        return hipStreamWaitEvent(c->stream, c->launch_done, 0) == hipSuccess;
+    c->launch_busy = hipEventQuery(c->launch_done) != hipSuccess;
+    (void)hipGetLastError();
+    return !c->launch_busy;
+}
+
 // Where a realization's visited-node bitmap lives (OKA_BITMAP_*, see
 // include/oka.h): a flat LDS bitmap when the whole grid fits in the LDS
 // budget beside the wells and window counters, else 32 x 32-node tiles in LDS
@@ -1078,8 +1107,10 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
     }
 
     // launch shape: a realization per workgroup of up to 256 lanes
+    const bool state = launch_state_free(c);
     const size_t base_lds =
-        (fp64 ? trace_fp64_wells_lds(a.nwells) : trace_fp32_wells_lds(a.nwells, a.confined)) +
+        (fp64 ? trace_fp64_wells_lds(a.nwells)
+              : trace_fp32_wells_lds(a.nwells, a.confined, state)) +
         win_lds;
     if (wells_limit_lds(a.nwells, fp64) + win_lds > c->max_lds)
         return fail(c, OKA_ERR_ARG, "too many wells for LDS (%d)", a.nwells);
@@ -1103,7 +1134,7 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
     const int nshared = std::min(nreal, std::min(resident, 5 * c->num_cu));   // 4 or 5 run at once
     const int spread = (int)std::min<int64_t>(
         c->num_cu, (int64_t)nreal * ((o->npaths - 1) / kTraceBlock + 1));
-    bool refills = !marks && o->npaths > kTraceBlock &&
+    bool refills = state && !marks && o->npaths > kTraceBlock &&
                    (int64_t)(words * 4) * (nshared + std::max(nshared, spread)) <= kMaxShareBytes;
     if (refills && words > 0) {
         if (ensure(c, kSlotShareBits, sizeof(uint32_t) * words * nshared, &o2) == OKA_OK) {
@@ -1114,7 +1145,7 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
             refills = false;
         }
     }
-    if (!marks && (refills || nreal > blocks)) {
+    if (state && !marks && (refills || nreal > blocks)) {
         blocks = refills ? std::max(nshared, spread) : std::min(nreal, resident);
         a.share_first = refills ? nreal - nshared : nreal;
         a.share_words = (int32_t)words;
@@ -1130,7 +1161,7 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
         if (kind == kBmTiled)   // overflow tiles start empty; each flush leaves them so
             TRY(fill_u32(c, a.gbitmap, (int64_t)words * blocks));
     }
-    if (!fp64) {   // grown in steps of 8,192 wells
+    if (!fp64 && state) {   // grown in steps of 8,192 wells
         TRY(ensure(c, kSlotWells32, sizeof(float2) * ((a.nwells + 8191) / 8192 * 8192), &o2));
         a.wells32 = (const float2 *)o2;
         HIPCHK(c, launch_site_wells32(a, (float2 *)o2, c->stream));
@@ -1143,8 +1174,18 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
         HIPCHK(c, launch_trace_fp32(a, blocks, kind, c->stream));
     if (timed)
         HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-    return chronicle_finish(c, a, rasterize, nnodes, ntr, counts, bbox, trace_status, trace_steps,
-                            stats, flags, win, marks, masks);
+    const bool kept = a.share || a.wells32;
+    const bool left_running = (flags & OKA_ASYNC) && (flags & OKA_PTR_DEVICE) && !stats;
+    if (kept && left_running) {
+        c->launch_busy = true;
+        c->launch_stream = c->stream;
+        HIPCHK(c, hipEventRecord(c->launch_done, c->stream));
+    }
+    TRY(chronicle_finish(c, a, rasterize, nnodes, ntr, counts, bbox, trace_status, trace_steps,
+                         stats, flags, win, marks, masks));
+    if (kept && !left_running)
+        c->launch_busy = false;
+    return OKA_OK;
 }
 
 // Copies a trace launch's outputs back (host buffers) and reads its statistics.
@@ -1261,7 +1302,7 @@ int oka_trace_chronicle_noalloc(oka_ctx *c, const oka_site *site, int32_t nreal,
 
     const bool fp64 = o->precision == OKA_FP64_EXACT;
     const size_t base_lds = fp64 ? trace_fp64_wells_lds(a.nwells)
-                                 : trace_fp32_wells_lds(a.nwells, a.confined);
+                                 : trace_fp32_wells_lds(a.nwells, a.confined, true);
     if (wells_limit_lds(a.nwells, fp64) > c->max_lds)
         return fail(c, OKA_ERR_ARG, "too many wells for LDS (%d)", a.nwells);
     int kind = kBmLdsFlat;

@@ -44,6 +44,12 @@ struct oka_ctx {
     int warp_size = 64;
     std::string err;
     oka::DevBuf buf[oka::kSlotCount];
+    // the workgroup tracers' launch state (kSlotShare, kSlotShareBits,
+    // kSlotWells32): whether a launch left running may still use it, on which
+    // stream, and its end
+    bool launch_busy = false;
+    hipStream_t launch_stream = nullptr;
+    hipEvent_t launch_done = nullptr;
     // device address of this device's copy of the no-allocation scratch
     // array (oka_trace_chronicle_noalloc), looked up at create; null if the
     // lookup failed, with its HIP error in scratch_err

@@ -19,15 +19,21 @@ using namespace fp32;
 // At most 128 VGPRs, so that at least 4 waves share a SIMD: the tracer is
 // bound by VALU issue, and with 3 waves the SIMDs idled about 12 % of the time
 // on LDS and scalar waits.
-template <int kKind, bool kConfined>
+//
+// kPlaces: the wells' places come from a.wells32 (Field32Site).  Without it,
+// where nothing outside the launch may hold them, they are records in LDS.
+template <int kKind, bool kConfined, bool kPlaces>
 __global__ void __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4)))
 k_trace_fp32(TraceArgs a)
 {
     extern __shared__ float4 smem4[];
-    // strengths, then (unconfined) the potential's, of 4 wells a float4
+    using Field = typename std::conditional<kPlaces, Field32Site, Field32Lds>::type;
+    // a record a well, or strengths, then (unconfined) the potential's, of 4
+    // wells a float4
     const int nw4 = (a.nwells + 3) / 4;
     float *s_q = reinterpret_cast<float *>(smem4), *s_p = reinterpret_cast<float *>(smem4 + nw4);
-    uint32_t *s_bm = reinterpret_cast<uint32_t *>(smem4 + (kConfined ? 1 : 2) * nw4);
+    uint32_t *s_bm = reinterpret_cast<uint32_t *>(
+        smem4 + (!kPlaces ? a.nwells : (kConfined ? 1 : 2) * nw4));
     using Bits = typename std::conditional<kKind == kBmTiled, TileBits, FlatBits>::type;
     __shared__ int s_next;
     __shared__ ShareLds s_share;
@@ -79,9 +85,16 @@ k_trace_fp32(TraceArgs a)
         const double h = kConfined ? 1.0 : 0.5 * a.K[r] * (a.b[r] * a.b[r]);
         for (int i = tid; i < a.nwells; i += blockDim.x) {
             const double qw = a.q[(int64_t)r * a.nwells + i];
-            s_q[i] = (float)(qw * kInv2Pi / bn);
-            if constexpr (!kConfined)
-                s_p[i] = (float)(qw * (kInv4Pi * kLn2) / h);
+            const float st = (float)(qw * kInv2Pi / bn);
+            const float pt = kConfined ? 0.0f : (float)(qw * (kInv4Pi * kLn2) / h);
+            if constexpr (kPlaces) {
+                s_q[i] = st;
+                if constexpr (!kConfined)
+                    s_p[i] = pt;
+            } else {
+                smem4[i] = make_float4((float)(a.wells_xy[2 * i] - a.xo),
+                                       (float)(a.wells_xy[2 * i + 1] - a.yo), st, pt);
+            }
         }
         if (tid == 0) {
             const double *c = a.coef + 6 * (int64_t)r;
@@ -101,10 +114,14 @@ k_trace_fp32(TraceArgs a)
         }
         __syncthreads();
 
-        Field32Site f;
-        f.xy = (ConstF32)a.wells32;
-        f.q4 = smem4;
-        f.p4 = smem4 + nw4;
+        Field f;
+        if constexpr (kPlaces) {
+            f.xy = (ConstF32)a.wells32;
+            f.q4 = smem4;
+            f.p4 = smem4 + nw4;
+        } else {
+            f.w = smem4;
+        }
         f.nw = a.nwells;
         f.a2 = s_reg[0];
         f.b2 = s_reg[1];
@@ -161,8 +178,8 @@ k_trace_fp32(TraceArgs a)
                 }
             } else {
                 float ox, oy;
-                const int res = finish32(LaneEval<kConfined, Field32Site>{f, dry}, I, s, dtd, dt, kx,
-                                         ky, ox, oy);
+                const int res = finish32(LaneEval<kConfined, Field>{f, dry}, I, s, dtd, dt, kx, ky,
+                                         ox, oy);
                 // a stage raised: the step is not accepted and the trace ends
                 if (!kConfined && dry)
                     s.status = OKA_TRACE_TRUNCATED;
@@ -244,9 +261,10 @@ __global__ void __launch_bounds__(256) k_raster_fp32(RasterArgs a)
 
 }  // namespace
 
-size_t trace_fp32_wells_lds(int nwells, bool confined)
+size_t trace_fp32_wells_lds(int nwells, bool confined, bool places)
 {
-    return (size_t)((nwells + 3) / 4) * sizeof(float4) * (confined ? 1 : 2);
+    return sizeof(float4) *
+           (!places ? (size_t)nwells : (size_t)((nwells + 3) / 4) * (confined ? 1 : 2));
 }
 
 hipError_t launch_site_wells32(const TraceArgs &a, float2 *out, hipStream_t s)
@@ -258,29 +276,36 @@ hipError_t launch_site_wells32(const TraceArgs &a, float2 *out, hipStream_t s)
     return hipGetLastError();
 }
 
+namespace {
+
+template <int kKind>
+hipError_t launch_kind(const TraceArgs &a, int grid_blocks, size_t lds, hipStream_t s)
+{
+    const dim3 grid(grid_blocks), block(trace_block(a.npaths));
+    if (a.confined && a.wells32)
+        hipLaunchKernelGGL((k_trace_fp32<kKind, true, true>), grid, block, lds, s, a);
+    else if (a.confined)
+        hipLaunchKernelGGL((k_trace_fp32<kKind, true, false>), grid, block, lds, s, a);
+    else if (a.wells32)
+        hipLaunchKernelGGL((k_trace_fp32<kKind, false, true>), grid, block, lds, s, a);
+    else
+        hipLaunchKernelGGL((k_trace_fp32<kKind, false, false>), grid, block, lds, s, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_trace_fp32(const TraceArgs &a, int grid_blocks, int kind, hipStream_t s)
 {
-    size_t lds = trace_fp32_wells_lds(a.nwells, a.confined) +
+    size_t lds = trace_fp32_wells_lds(a.nwells, a.confined, a.wells32 != nullptr) +
                  (a.wmarks ? (size_t)a.w_nr * a.w_nc * 4 : 0);
-    dim3 grid(grid_blocks), block(trace_block(a.npaths));
-    if (!a.rasterize || kind == kBmLdsFlat) {
-        lds += a.rasterize ? (size_t)a.nwords * 4 : 0;
-        if (a.confined)
-            hipLaunchKernelGGL((k_trace_fp32<kBmLdsFlat, true>), grid, block, lds, s, a);
-        else
-            hipLaunchKernelGGL((k_trace_fp32<kBmLdsFlat, false>), grid, block, lds, s, a);
-    } else if (kind == kBmTiled) {
-        lds += (size_t)tile_lds_words(a.ntiles, a.tile_slots) * 4;
-        if (a.confined)
-            hipLaunchKernelGGL((k_trace_fp32<kBmTiled, true>), grid, block, lds, s, a);
-        else
-            hipLaunchKernelGGL((k_trace_fp32<kBmTiled, false>), grid, block, lds, s, a);
-    } else if (a.confined) {
-        hipLaunchKernelGGL((k_trace_fp32<kBmHbmFlat, true>), grid, block, lds, s, a);
-    } else {
-        hipLaunchKernelGGL((k_trace_fp32<kBmHbmFlat, false>), grid, block, lds, s, a);
-    }
-    return hipGetLastError();
+    if (!a.rasterize || kind == kBmLdsFlat)
+        return launch_kind<kBmLdsFlat>(a, grid_blocks,
+                                       lds + (a.rasterize ? (size_t)a.nwords * 4 : 0), s);
+    if (kind == kBmTiled)
+        return launch_kind<kBmTiled>(
+            a, grid_blocks, lds + (size_t)tile_lds_words(a.ntiles, a.tile_slots) * 4, s);
+    return launch_kind<kBmHbmFlat>(a, grid_blocks, lds, s);
 }
 
 hipError_t launch_raster_fp32(const RasterArgs &a, hipStream_t s)

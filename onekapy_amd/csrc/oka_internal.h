@@ -65,7 +65,7 @@ struct TraceArgs {
     int32_t nwells;
     int32_t npaths;
     const double *wells_xy;     // nwells x 2
-    const float2 *wells32;      // FP32 workgroup tracer: wells_xy - (xo, yo)
+    const float2 *wells32;      // FP32 workgroup tracer: wells_xy - (xo, yo), or nullptr
     const double *start_xy;     // npaths x 2
     double xo, yo;
     // realizations
@@ -650,7 +650,7 @@ size_t trace_fp64_wells_lds(int nwells);
 // oka_fp32.hip
 hipError_t launch_trace_fp32(const TraceArgs &a, int grid_blocks, int kind,
                              hipStream_t s);
-size_t trace_fp32_wells_lds(int nwells, bool confined);
+size_t trace_fp32_wells_lds(int nwells, bool confined, bool places);
 // TraceArgs::wells32 of the site of `a`, to out [nwells].
 hipError_t launch_site_wells32(const TraceArgs &a, float2 *out, hipStream_t s);
 

@@ -479,7 +479,8 @@ int check_opts(oka_ctx *c, const oka_trace_opts *o)
 constexpr int64_t kDefaultMaxSteps = 1000000;
 
 // Most memory for the merged bitmaps of shared realizations and the overflow
-// regions beside them.
+// regions beside them, which the context keeps until it is destroyed; ensure's
+// spare quarter counts.
 constexpr int64_t kMaxShareBytes = 2ll << 30;
 
 // The workgroup schedule takes as many wells as whole records of them (32
@@ -920,6 +921,18 @@ int run_pool(oka_ctx *c, const TraceArgs *sites, int nsites, const oka_trace_opt
     return OKA_OK;
 }
 
+// ensure() for memory that the call can do without: a failure leaves nothing
+// to report.
+bool try_ensure(oka_ctx *c, Slot s, size_t bytes, void **out)
+{
+    const std::string err = c->err;
+    if (ensure(c, s, bytes, out) == OKA_OK)
+        return true;
+    (void)hipGetLastError();
+    c->err = err;
+    return false;
+}
+
 // Whether this call may keep launch state in the context's slots (the queue,
 // the merged bitmaps, the FP32 wells' places): not while a launch on another
 // stream may still be using it, and not under capture, whose graph would hold
@@ -1125,28 +1138,29 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
     const int per_cu =
         (int)std::max<size_t>(1, std::min<size_t>(8, c->lds_per_cu / std::max<size_t>(lds, 1)));
     const int resident = c->num_cu * per_cu;   // or more than the registers let run
-    int blocks = kind == kBmLdsFlat ? nreal : std::min(nreal, resident);
+    const int nshared = std::min(nreal, std::min(resident, 5 * c->num_cu));   // 4 or 5 run at once
+    int blocks = kind == kBmLdsFlat           ? nreal
+                 : o->npaths > kTraceBlock ? nshared
+                                           : std::min(nreal, resident);
     // Realizations are taken from a queue where a workgroup has several, and
     // the last ones shared (next_realization) where their particles outnumber
     // a workgroup's lanes; few realizations then get workgroups for all their
     // particles.  The window marks belong to one workgroup, and without the
     // memory for the merged bitmaps nothing is shared.
-    const int nshared = std::min(nreal, std::min(resident, 5 * c->num_cu));   // 4 or 5 run at once
     const int spread = (int)std::min<int64_t>(
         c->num_cu, (int64_t)nreal * ((o->npaths - 1) / kTraceBlock + 1));
     bool refills = state && !marks && o->npaths > kTraceBlock &&
-                   (int64_t)(words * 4) * (nshared + std::max(nshared, spread)) <= kMaxShareBytes;
+                   (int64_t)(words * 5) * (nshared + std::max(nshared, spread)) <= kMaxShareBytes;
     if (refills && words > 0) {
-        if (ensure(c, kSlotShareBits, sizeof(uint32_t) * words * nshared, &o2) == OKA_OK) {
+        refills = try_ensure(c, kSlotShareBits, sizeof(uint32_t) * words * nshared, &o2);
+        if (refills) {
             a.share_bits = (uint32_t *)o2;
             TRY(fill_u32(c, a.share_bits, (int64_t)words * nshared));
-        } else {
-            (void)hipGetLastError();
-            refills = false;
         }
     }
     if (state && !marks && (refills || nreal > blocks)) {
-        blocks = refills ? std::max(nshared, spread) : std::min(nreal, resident);
+        if (refills)
+            blocks = std::max(nshared, spread);
         a.share_first = refills ? nreal - nshared : nreal;
         a.share_words = (int32_t)words;
         const size_t counters = kShareStride * (1 + (size_t)(nreal - a.share_first));
@@ -1155,7 +1169,11 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
         TRY(fill_u32(c, a.share, (int64_t)counters));
     }
     if (kind != kBmLdsFlat) {
-        // per-workgroup HBM regions, of the workgroups that the LDS lets run at once
+        // per-workgroup HBM regions, of the workgroups that can run at once or,
+        // when memory is short, of fewer
+        while (blocks > 2 * c->num_cu &&
+               !try_ensure(c, kSlotBitmap, sizeof(uint32_t) * words * blocks, &o2))
+            blocks /= 2;
         TRY(ensure(c, kSlotBitmap, sizeof(uint32_t) * words * blocks, &o2));
         a.gbitmap = (uint32_t *)o2;
         if (kind == kBmTiled)   // overflow tiles start empty; each flush leaves them so

@@ -60,10 +60,10 @@ class Launches:
         ds.counts = self.mem.put(np.zeros(ds.shape, np.int32))
         return ds
 
-    def launch(self, ds, precision, flags=_lib.PTR_DEVICE | _lib.ASYNC):
+    def launch(self, ds, precision, flags=_lib.PTR_DEVICE | _lib.ASYNC, **kw):
         opts = _lib.make_trace_opts(ds.P, ds.s.duration, ds.s.tol, ds.s.maxstep, ds.umbra,
                                     ds.starts, precision, True,
-                                    schedule=_lib.SCHED_WORKGROUP)
+                                    schedule=_lib.SCHED_WORKGROUP, **kw)
         self.ctx.check(self.ctx.lib.oka_trace_chronicle(
             self.ctx.h, C.byref(ds.site), ds.nreal, ds.K, ds.n, ds.b, ds.q, ds.coef,
             C.byref(opts), C.byref(ds.grid), 1, ds.epoch, 1, ds.counts, None, None, None, None,
@@ -76,9 +76,9 @@ class Launches:
     def counts(self, ds):
         return self.mem.get(ds.counts, ds.shape, np.int32)
 
-    def alone(self, ds, precision):
+    def alone(self, ds, precision, **kw):
         """The counts of a synchronous launch with nothing else running."""
-        self.launch(ds, precision, _lib.PTR_DEVICE)
+        self.launch(ds, precision, _lib.PTR_DEVICE, **kw)
         out = self.counts(ds)
         self.clear(ds)
         assert out.any()
@@ -144,5 +144,27 @@ def test_captured_launch_outlives_larger_calls(launches, precision):
         n = (k > 0) + (k == 2)
         assert np.array_equal(launches.counts(big), n * want_big), k
         launches.clear(big)
+    launches.do("hipGraphExecDestroy", ex)
+    launches.do("hipGraphDestroy", graph)
+
+
+@PRECISIONS
+def test_captured_launch_needs_no_more_memory_than_its_warm_up(launches, precision):
+    """Bitmaps in HBM, more realizations than workgroups at once: the regions of
+    the captured launch are no larger than those of the eager one before it."""
+    ds = launches.site(0, 2500, 260, 40.0, 100)
+    want = launches.alone(ds, precision, bitmap_mode=_lib.BITMAP_HBM_FLAT)
+    s = launches.stream()
+    launches.ctx.set_stream(s)
+    graph, ex = C.c_void_p(), C.c_void_p()
+    launches.do("hipStreamBeginCapture", s, 2)   # relaxed
+    launches.launch(ds, precision, bitmap_mode=_lib.BITMAP_HBM_FLAT)
+    launches.do("hipStreamEndCapture", s, C.byref(graph))
+    launches.do("hipGraphInstantiate", C.byref(ex), graph, None, None, 0)
+    for k in range(3):
+        launches.do("hipGraphLaunch", ex, s)
+        launches.do("hipStreamSynchronize", s)
+        assert np.array_equal(launches.counts(ds), want), k
+        launches.clear(ds)
     launches.do("hipGraphExecDestroy", ex)
     launches.do("hipGraphDestroy", graph)

@@ -49,8 +49,12 @@ def impact_curve(spacing, pf):
     if pf.total_weight <= 0:
         raise CaptureZoneError('Empty capture zone')
     pr = sorted_probabilities(pf.pgrid, pf.total_weight)
-    area = np.arange(1.0, pr.shape[0] + 1.0)
-    area *= spacing ** 2
+    cell = spacing ** 2
+    if isinstance(cell, float):
+        area = np.arange(1.0, pr.shape[0] + 1.0)
+        area *= cell
+    else:   # whole spacings have whole areas
+        area = np.arange(1, pr.shape[0] + 1) * cell
     return pr, area
 
 

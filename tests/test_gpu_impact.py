@@ -79,6 +79,14 @@ def test_impact_curve_of_weighted_fields_equals_numpy_sort(gpu_ctx):
         assert np.array_equal(got, np.flip(np.sort(g / tw, axis=None))), shape
 
 
+@pytest.mark.parametrize("spacing", [20, 20.0, np.float32(2.5), np.int32(3), np.float64(0.1)])
+def test_impact_curve_area_has_the_spacings_type(gpu_ctx, spacing):
+    ref = np.load(os.path.join(GOLDEN, "reference_impact.npz"))
+    _, area = impact_curve(spacing, _field(ref["counts"], 37.0))
+    want = (np.arange(ref["counts"].size) + 1) * spacing ** 2
+    assert area.dtype == want.dtype and np.array_equal(area, want)
+
+
 @pytest.mark.parametrize("smooth", [0.0, 0.5, 1.0, 2.0, 3.7, 8.0])
 def test_smoothed_probability_equals_scipy(gpu_ctx, smooth):
     """Pr = pgrid / total_weight and its Gaussian smoothing (sigma in nodes,

@@ -9,7 +9,9 @@ The GPU sorts the probabilities (oka_field_sorted_probabilities): with weight 1
 per realization (stochastic.py:265) pgrid holds integer counts and the sort is
 a counting sort, any other field (weights other than 1, e.g.
 compute_capturezone's weight argument) is radix-sorted; both give the same
-array as numpy's sort, value for value.
+array as numpy's sort, value for value.  A field of integer counts with more
+nodes than that sort takes is laid out from the GPU histogram of its counts
+(oka_count_histogram).
 """
 import math
 
@@ -18,6 +20,7 @@ import numpy as np
 from . import _lib
 
 ACRE_M2 = 4046.86   # m^2 per acre (visualize.py:387, oneka.py:288)
+MAX_SORTED_NODES = 2 ** 31 - 1   # oka_field_sorted_probabilities' limit
 
 
 class CaptureZoneError(Exception):
@@ -48,7 +51,19 @@ def impact_curve(spacing, pf):
     """(pr, area) as create_impact_plot returns them (visualize.py:382-385)."""
     if pf.total_weight <= 0:
         raise CaptureZoneError('Empty capture zone')
-    pr = sorted_probabilities(pf.pgrid, pf.total_weight)
+    counts = None
+    if np.size(pf.pgrid) > MAX_SORTED_NODES:
+        counts = np.rint(pf.pgrid)
+        if not (np.array_equal(counts, pf.pgrid) and counts.min() >= 0 and
+                counts.max() < 2 ** 31):
+            counts = None
+    if counts is None:
+        pr = sorted_probabilities(pf.pgrid, pf.total_weight)
+    else:
+        top = int(counts.max())
+        hist = count_histogram(counts.astype(np.int32), top)
+        values = np.arange(top, -1, -1, dtype=np.float64) / pf.total_weight   # descending
+        pr = np.repeat(values, hist[::-1])
     cell = spacing ** 2
     if isinstance(cell, float):
         area = np.arange(1.0, pr.shape[0] + 1.0)

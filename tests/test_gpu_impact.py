@@ -1,5 +1,5 @@
-"""Impact curve and deciles (GPU count histogram, or GPU radix sort for
-fields of other weights) against the reference's create_impact_plot values
+"""Impact curve and deciles (GPU counting sort of whole counts, or GPU radix
+sort for fields of other weights) against the reference's create_impact_plot values
 and oneka()'s decile rows, and the smoothed probability map against
 scipy.ndimage.gaussian_filter (visualize.py:232-233)."""
 import os
@@ -50,7 +50,7 @@ def test_impact_curve_edge_cases(gpu_ctx):
     ref = np.load(os.path.join(GOLDEN, "reference_impact.npz"))
     with pytest.raises(CaptureZoneError):
         impact_curve(20.0, _field(ref["counts"], 0.0))
-    # a field of weight-0.5 realizations is sorted as a whole (no histogram)
+    # a field of weight-0.5 realizations is radix-sorted
     pr, _ = impact_curve(20.0, _field(ref["counts"] * 0.5, 37.0))
     assert np.array_equal(pr, np.flip(np.sort(ref["counts"] * 0.5 / 37.0, axis=None)))
     # every node certain
@@ -77,6 +77,23 @@ def test_impact_curve_of_weighted_fields_equals_numpy_sort(gpu_ctx):
         g[rng.random(shape) < 0.6] = 0.0
         got = sorted_probabilities(g, tw)
         assert np.array_equal(got, np.flip(np.sort(g / tw, axis=None))), shape
+
+
+@pytest.mark.parametrize("whole", [True, False])
+def test_impact_curve_of_more_nodes_than_the_sort_takes(gpu_ctx, monkeypatch, whole):
+    """Whole counts go through the histogram (the limit lowered: 2^31 nodes are
+    16 GiB); any other field is the sort's to refuse."""
+    from onekapy_amd import impact
+    ref = np.load(os.path.join(GOLDEN, "reference_impact.npz"))
+    pf = _field(ref["counts"] * (1.0 if whole else 0.5), 37.0)
+    want, area = impact_curve(20.0, pf)
+    sorts = []
+    monkeypatch.setattr(impact, "MAX_SORTED_NODES", pf.pgrid.size - 1)
+    monkeypatch.setattr(impact, "sorted_probabilities",
+                        lambda *a: sorts.append(a) or sorted_probabilities(*a))
+    pr, got = impact_curve(20.0, pf)
+    assert len(sorts) == (0 if whole else 1)
+    assert np.array_equal(pr, want) and np.array_equal(got, area)
 
 
 @pytest.mark.parametrize("spacing", [20, 20.0, np.float32(2.5), np.int32(3), np.float64(0.1)])

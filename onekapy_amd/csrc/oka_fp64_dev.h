@@ -136,11 +136,19 @@ __device__ __forceinline__ double recip_plain(double b)
 // next to a / b, the residual a - b q0 is exact, and q0 + residual r lies
 // within 2^-107 m (1 + 2^-16) (times the exponent of the quotient) of a / b.
 // A quotient differs from a rounding boundary by at least 2^-105 / m, so the
-// final rounding is that of a / b for every m < 2 - 2^-16 (above it only
-// numerators within 2^-53 of the worst case could differ, as in the
-// compiler's own sequence at m = 2 - 2^-52).  The residual is formed negated,
-// b q0 - a, so that a zero numerator keeps its sign through the sum
-// (-(+0) r + (-0) = -0) and no div_fixup is needed.  0 / 0 gives NaN: r0 is
+// final rounding is that of a / b for every m < 2 - 2^-16.  Above it the proof
+// needs r to be the double nearest to 1 / b.  There b is 2 - k 2^-52 (times a
+// power of two) and 1 / b, for odd k, lies a relative k^2 2^-106 above the
+// middle of two doubles, which the e0^3 that recip_plain leaves out could reach for k below
+// 2^16.6.  But the hardware's estimate is then above 1 / b (it is one value for
+// k = 2 to 2^20), so leaving out e0^3 < 0 errs upwards, and r is the upper of
+// the two, the nearer one: checked on the GPU for every k up to 2^20 and six
+// exponents.  (Two Newton steps give the lower one for k = 3, 5 .. 13, and the
+// other double for some numerators of k = 5, 11 and 13.)  With the nearer r the
+// quotients of the 32,080 numerators closest to a boundary, for the odd k up to
+// 4,000 and four larger ones, are those of exact arithmetic.  The residual is
+// formed negated, b q0 - a, so that a zero numerator keeps its sign through the
+// sum (-(+0) r + (-0) = -0) and no div_fixup is needed.  0 / 0 gives NaN: r0 is
 // infinite and e0 NaN.
 __device__ __forceinline__ double quot_plain(double a, double b, double r)
 {
@@ -638,10 +646,16 @@ __device__ __forceinline__ void raster_node(Bits &bits, const EpochReg &e, const
 // Most of a window's nodes lie outside the umbra or are marked already, so
 // each row first takes, in float, the chord of the capsule around the segment
 // at a radius 2^-10 larger than umbra (raster32's, with its clip widened by as
-// much), which contains every node the exact test could mark: the float
-// errors are below 2^-20 of the umbra for segments up to 1,000 umbras.  Only
-// its unmarked nodes, read a word at a time, take the exact test.  Against the
-// exact test at every unmarked node of the window: 10^4 x 1000 particles of
+// much), which contains every node the exact test could mark.  The widening is
+// sized for segments of up to 1,000 umbras: a float coordinate of 1,000 umbras
+// is rounded by 2^-14 umbras, the row's offset c carries up to three such
+// errors, and with those of the slopes and of the columns the band's sides are
+// off by at most three quarters of the 2^-10.  The end lines may be off by a
+// little more than all of it, but the discs around the ends, off by less than a
+// quarter, hold the nodes that this could cost.  (A replay of the arithmetic on
+// 4e7 nodes inside the umbra, segments up to 998 umbras: c off by 2^-13, no
+// node lost.)  Only the chord's unmarked nodes, read a word at a time, take the
+// exact test.  Against the exact test at every unmarked node of the window: 10^4 x 1000 particles of
 // the 25-well site 126.2 -> 119.9 ms, 100 x 100 of the 4-well site 14 % less.
 template <typename Bits>
 __device__ __forceinline__ int raster_segment(Bits &bits, const EpochReg &e, const Raster64 &g,
@@ -679,6 +693,7 @@ __device__ __forceinline__ int raster_segment(Bits &bits, const EpochReg &e, con
     const int ncand = (j1 - j0) * (i1 - i0);
     // the row's chord: x - ax in (lo, hi) with c = y_row - ay; in columns from j0
     const float fbx = (float)bax, fby = (float)bay, fl2 = (float)l2;
+    // the length's limit and g.slack depend on each other
     const bool chord = g.fast && fabsf(fbx) > 1e-20f && fabsf(fby) > 1e-20f &&
                        fl2 < 1e6f * g.outer2 && j1 - j0 < 4096 && i1 - i0 < 4096;
     const float ibx = __builtin_amdgcn_rcpf(fbx), iby = __builtin_amdgcn_rcpf(fby);

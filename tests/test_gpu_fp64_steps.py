@@ -67,3 +67,39 @@ def test_step_factor_rules_bit_exact_vs_oracle(gpu_ctx, tol, maxstep):
                                max_steps=cap)
         assert (status[0], nverts[0]) == (res.status, res.nverts)
         assert np.array_equal(verts[0, :nverts[0]], ov)
+
+
+def _worst_numerators(k):
+    """Mantissas (of 53 bits) whose quotients by b = 2 - k 2^-52 lie closest to
+    the middle of two doubles: 2^54 A = r (mod 2^53 - k) for small odd r."""
+    b = 2 ** 53 - k
+    inv = pow(2 ** 54, -1, b)
+    out = [r * inv % b for r in (1, -1, 3, -3, 5, -5, 7, -7)]
+    return [a for a in out if a > b // 2]
+
+
+def test_quotients_by_divisors_just_below_a_power_of_two(gpu_ctx):
+    """thickness x porosity = 2 - k 2^-52 for odd k, where a reciprocal that is
+    not the nearest double gives the wrong quotient for the numerators used
+    here, the regional discharges: the vertices are the oracle's, whose
+    division is IEEE's."""
+    cases = [(k, a) for k in (1, 3, 5, 7, 9, 11, 13, 25, 33, 35, 999, 4001, 65535, 65537)
+             for a in _worst_numerators(k)]
+    # numerators a * 2^-52 and, along y, the next case's
+    d = np.array([a * 2.0 ** -52 for _, a in cases])
+    thick = np.array([(2 ** 53 - k) * 2.0 ** -51 for k, _ in cases])
+    e = np.array([cases[(i + 1) % len(cases)][1] * -2.0 ** -53
+                  if cases[(i + 1) % len(cases)][0] == k else 0.0
+                  for i, (k, _) in enumerate(cases)])
+    n = len(cases)
+    w = np.array([(500.0, 300.0, 0.25, 0.0)])
+    coef = np.zeros((n, 6))
+    coef[:, 3], coef[:, 4] = d, e
+    real = Realizations(np.full(n, 10.0), np.full(n, 0.5), thick, np.zeros((n, 1)), coef)
+    verts, nverts, status = trace_vertices(np.ascontiguousarray(w[:, :2]), 0.0, 0.0, real,
+                                           np.zeros((1, 2)), 50.0, 1.0, 10.0, True, 40)
+    for i, (k, _) in enumerate(cases):
+        om = O.OracleModel(0.0, 10.0, 0.5, thick[i], w, 0.0, 0.0, tuple(coef[i]))
+        ov, res = om.backtrace(0.0, 0.0, 50.0, 1.0, 10.0, confined=True, max_steps=40)
+        assert (status[i], nverts[i]) == (res.status, res.nverts), k
+        assert np.array_equal(verts[i, :nverts[i]], ov), k

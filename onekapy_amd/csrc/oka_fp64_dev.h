@@ -84,6 +84,38 @@ struct FieldSite : Field64 {
     }
 };
 
+// a1 / b and a2 / b, each correctly rounded (IEEE division, as numpy's).
+// gfx950 has no division instruction; the compiler expands every FP64 `/`
+// into one fixed sequence:
+//   d = div_scale(b; b, a)  r = rcp(d)  r += r (1 - d r)  r += r (1 - d r)
+//   n, s = div_scale(a; b, a)  m = n r  q = div_fmas(fma(-d, m, n), r, m; s)
+//   q = div_fixup(q, b, a)
+// Only d and r depend on the numerator, through d's scaling of extreme
+// exponents.  When both numerators leave d the same (always, in the normal
+// range), this runs that sequence once for d and r and twice for the rest,
+// so each result has the bits `a / b` would have; otherwise it divides twice.
+__device__ __forceinline__ void div_pair(double a1, double a2, double b, double &q1, double &q2)
+{
+    bool s1, s2;
+    const double d = __builtin_amdgcn_div_scale(a1, b, false, &s1);
+    const double d2 = __builtin_amdgcn_div_scale(a2, b, false, &s2);
+    if (__double_as_longlong(d) != __double_as_longlong(d2)) {
+        q1 = a1 / b;
+        q2 = a2 / b;
+        return;
+    }
+    double r = __builtin_amdgcn_rcp(d);
+    r = fma(r, fma(-d, r, 1.0), r);
+    r = fma(r, fma(-d, r, 1.0), r);
+    const double n1 = __builtin_amdgcn_div_scale(a1, b, true, &s1);
+    const double n2 = __builtin_amdgcn_div_scale(a2, b, true, &s2);
+    const double m1 = n1 * r, m2 = n2 * r;
+    q1 = __builtin_amdgcn_div_fixup(
+        __builtin_amdgcn_div_fmas(fma(-d, m1, n1), r, m1, s1), b, a1);
+    q2 = __builtin_amdgcn_div_fixup(
+        __builtin_amdgcn_div_fmas(fma(-d, m2, n2), r, m2, s2), b, a2);
+}
+
 // 1 / b for a divisor that needs no scaling (see plain_coord): the hardware
 // estimate r0 (relative error e0 below 2^-23, measured 2^-24.3 at most over
 // 4e9 divisors) and one third-order step, r0 (1 + e0 + e0^2), whose error
@@ -96,38 +128,6 @@ __device__ __forceinline__ double recip_plain(double b)
     const double r0 = __builtin_amdgcn_rcp(b);
     const double e = fma(-b, r0, 1.0);
     return fma(r0, fma(e, e, e), r0);
-}
-
-// a1 / b and a2 / b, each correctly rounded (IEEE division, as numpy's).
-// gfx950 has no division instruction; the compiler expands every FP64 `/`
-// into one fixed sequence:
-//   d = div_scale(b; b, a)  r = rcp(d)  r += r (1 - d r)  r += r (1 - d r)
-//   n, s = div_scale(a; b, a)  m = n r  q = div_fmas(fma(-d, m, n), r, m; s)
-//   q = div_fixup(q, b, a)
-// Only d and r depend on the numerator, through d's scaling of extreme
-// exponents.  When both numerators leave d the same (always, in the normal
-// range), this runs that sequence once for d and r and twice for the rest;
-// otherwise it divides twice.  r is recip_plain's, which is nearer than two
-// Newton steps for some divisors just below a power of two (see quot_plain);
-// for those `/` is not quite correctly rounded.
-__device__ __forceinline__ void div_pair(double a1, double a2, double b, double &q1, double &q2)
-{
-    bool s1, s2;
-    const double d = __builtin_amdgcn_div_scale(a1, b, false, &s1);
-    const double d2 = __builtin_amdgcn_div_scale(a2, b, false, &s2);
-    if (__double_as_longlong(d) != __double_as_longlong(d2)) {
-        q1 = a1 / b;
-        q2 = a2 / b;
-        return;
-    }
-    const double r = recip_plain(d);
-    const double n1 = __builtin_amdgcn_div_scale(a1, b, true, &s1);
-    const double n2 = __builtin_amdgcn_div_scale(a2, b, true, &s2);
-    const double m1 = n1 * r, m2 = n2 * r;
-    q1 = __builtin_amdgcn_div_fixup(
-        __builtin_amdgcn_div_fmas(fma(-d, m1, n1), r, m1, s1), b, a1);
-    q2 = __builtin_amdgcn_div_fixup(
-        __builtin_amdgcn_div_fmas(fma(-d, m2, n2), r, m2, s2), b, a2);
 }
 
 // a / b correctly rounded from r = recip_plain(b), for operands that need no

@@ -479,9 +479,9 @@ int check_opts(oka_ctx *c, const oka_trace_opts *o)
 constexpr int64_t kDefaultMaxSteps = 1000000;
 
 // Most memory for the merged bitmaps of shared realizations and the overflow
-// regions beside them, which the context keeps until it is destroyed; ensure's
-// spare quarter counts.
-constexpr int64_t kMaxShareBytes = 2ll << 30;
+// regions beside them, ensure's spare quarter included (2.5 GiB).  The context
+// keeps it until it is destroyed.
+constexpr int64_t kMaxShareBytes = 5ll << 29;
 
 // The workgroup schedule takes as many wells as whole records of them (32
 // bytes in FP64, 16 in FP32) fit in a workgroup's LDS.

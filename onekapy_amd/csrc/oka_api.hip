@@ -935,15 +935,16 @@ bool try_ensure(oka_ctx *c, Slot s, size_t bytes, void **out)
 
 // Whether this call may keep launch state in the context's slots (the queue,
 // the merged bitmaps, the FP32 wells' places): not while a launch on another
-// stream may still be using it, and not under capture, whose graph would hold
-// their addresses after they have grown.  Such a call launches a workgroup a
+// stream may still be using it, and not under capture (which only a call that
+// is left running can be), whose graph would hold their addresses after they
+// have grown.  Such a call launches a workgroup a
 // realization, with the wells' records in its LDS: 10^4 x 1000 particles of the
 // benchmark's 25-well site FP64 169.4 ms instead of 164.3, FP32 57.1 instead
 // of 51.1.
-bool launch_state_free(oka_ctx *c)
+bool launch_state_free(oka_ctx *c, bool left_running)
 {
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &capture) != hipSuccess) {
+    if (left_running && hipStreamIsCapturing(c->stream, &capture) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
@@ -1120,7 +1121,8 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
     }
 
     // launch shape: a realization per workgroup of up to 256 lanes
-    const bool state = launch_state_free(c);
+    const bool left_running = (flags & OKA_ASYNC) && (flags & OKA_PTR_DEVICE) && !stats;
+    const bool state = launch_state_free(c, left_running);
     const size_t base_lds =
         (fp64 ? trace_fp64_wells_lds(a.nwells)
               : trace_fp32_wells_lds(a.nwells, a.confined, state)) +
@@ -1193,7 +1195,6 @@ int chronicle_impl(oka_ctx *c, const oka_site *site, int32_t nreal, const double
     if (timed)
         HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     const bool kept = a.share || a.wells32;
-    const bool left_running = (flags & OKA_ASYNC) && (flags & OKA_PTR_DEVICE) && !stats;
     if (kept && left_running) {
         c->launch_busy = true;
         c->launch_stream = c->stream;

@@ -33,7 +33,7 @@
 // observations on, and the solve's chains are then hardly overlapped.  10^5
 // realizations of 200 wells and 200 observations: 6.48 ms with one lane per
 // realization doing everything (each wave's loads of q in 64 rows, the
-// potentials summed twice), 1.36 ms so, 0.53 of them the solve.
+// potentials summed twice), 1.27 ms so, of which the solve takes about 0.5.
 #include <math.h>
 
 #include <algorithm>
@@ -646,10 +646,10 @@ size_t fit_lds_bytes(int nobs)
 
 // Two workgroups per CU where their LDS fits one (up to about 90
 // observations) and there are enough of them to share CUs: 10^5 realizations
-// of 200 wells and 64 observations 0.43 against 0.54 ms.  Alone on its CU a
+// of 200 wells and 64 observations 0.40 against 0.49 ms.  Alone on its CU a
 // workgroup is faster without the register limit, whose spills lengthen the
-// solve: 200 observations 1.42 against 1.64 ms, 100 realizations 31 against
-// 36 us.
+// solve: 200 observations 1.27 against 1.56 ms, 100 realizations of 25 wells
+// and 40 observations 32 against 37 us.
 bool fit_two(int nobs, int64_t blocks)
 {
     int dev = 0, num_cu = 0, lds = 0;

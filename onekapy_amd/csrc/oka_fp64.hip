@@ -75,11 +75,11 @@ struct Chron<kModeVertices> {
 // refilled from the LDS counter s_next, or the shared counter of one of the last
 // realizations, when their trace ends.
 // Both tracers are held to 128 VGPRs (4 waves per SIMD).  The confined one
-// spills one 64-bit value, stored before the realization loop and read after
-// it, and is 3 % faster than with the 150 the compiler picks.  The unconfined
-// one spills 256 bytes per lane but runs 13 % faster than with the 219 VGPRs
-// (2 waves per SIMD) the compiler picks: its correctly rounded logarithms
-// wait on table loads, which more waves hide.
+// spills 24 to 42 of them, by its bitmap; when it spilled two it was 3 % faster
+// than with the 150 the compiler picked.  The unconfined one spills about 150
+// (272 bytes a lane, 256 when it ran 13 % faster than with the 219 VGPRs, 2
+// waves per SIMD, the compiler picked): its correctly rounded logarithms wait
+// on table loads, which more waves hide.
 template <bool kConfined, int kMode>
 __global__ void __launch_bounds__(kTraceBlock)
 __attribute__((amdgpu_waves_per_eu(4))) k_trace_fp64(TraceArgs a)

@@ -84,8 +84,10 @@ struct FieldSite : Field64 {
     }
 };
 
-// a1 / b and a2 / b, each correctly rounded (IEEE division, as numpy's).
-// gfx950 has no division instruction; the compiler expands every FP64 `/`
+// a1 / b and a2 / b as the compiler divides: correctly rounded (IEEE division,
+// as numpy's) but for some numerators of the divisors with mantissa 2 - k 2^-52,
+// k = 5, 11 and 13 (see quot_plain; recip_plain's step here too would mend
+// those and costs the tiled tracers 2 %).  gfx950 has no division instruction; the compiler expands every FP64 `/`
 // into one fixed sequence:
 //   d = div_scale(b; b, a)  r = rcp(d)  r += r (1 - d r)  r += r (1 - d r)
 //   n, s = div_scale(a; b, a)  m = n r  q = div_fmas(fma(-d, m, n), r, m; s)
@@ -339,8 +341,9 @@ __device__ __forceinline__ bool feval(const F &f, double x, double y, double &kx
 
 // One field evaluation of every active lane: with the short sequences, and
 // again without them when the field or any lane's point does not allow them.
-// Both give the same bits where they apply, so one such lane may take its
-// wave along, and the long sequence stays off the usual path.
+// Both give the same bits where they apply (but for div_pair's exception), so
+// one such lane may take its wave along, and the long sequence stays off the
+// usual path.
 template <bool kConfined, class F>
 __device__ __forceinline__ bool eval64(const F &f, double x, double y, double &kx, double &ky)
 {

@@ -29,11 +29,11 @@ constexpr int kTileEmpty = -1, kTileOverflow = -2;
 constexpr int kMinTileSlots = 16;
 // Tile slots from which on more workgroups per CU are worth more than more
 // slots.  25 wells, 2 workgroups a CU (56 KiB each) -> the rule: 1600 x 1600 nodes,
-// 1,000 realizations x 1,000 particles (4 a CU, 229 slots) FP64 19.5 -> 17.7 ms, FP32
-// 8.2 -> 6.1; 4,000 x 100 (6 a CU, 122 slots) 21.7 -> 13.2 and 8.4 -> 5.0;
-// 8,000 x 30 36.0 -> 16.8 and 14.7 -> 7.0; 3000 x 3000, 1,000 x 1,000 (3 a CU, 132
-// slots) 34.6 -> 31.3 and 14.7 -> 11.9.  Below, tiles overflow into HBM: 3400 x
-// 3400 FP32 with 60 slots at 3 a CU 21.5 ms against 14.7 with 85 at 2.
+// 1,000 realizations x 1,000 particles (4 a CU, 229 slots) FP64 19.8 -> 17.2 ms, FP32
+// 8.2 -> 6.0; 4,000 x 100 (6 a CU, 122 slots) 21.9 -> 13.1 and 8.4 -> 5.1;
+// 8,000 x 30 36.5 -> 17.1 and 14.9 -> 7.0; 3000 x 3000, 1,000 x 1,000 (3 a CU, 132
+// slots) 38.9 -> 31.0 and 15.6 -> 12.0.  Below, tiles overflow into HBM: 3400 x
+// 3400 FP32 with 60 slots at 3 a CU 21.6 ms against 15.8 with 85 at 2.
 constexpr int kEnoughTileSlots = 96;
 constexpr size_t kLdsGrain = 2048;          // LDS is given out in steps no larger than this
 constexpr size_t kLdsOwn = 256;             // the trace kernels' own LDS variables, at most
@@ -354,10 +354,11 @@ __device__ __forceinline__ int claim_one(int32_t *counter)
 // empty therefore joins the realization with the most particles not yet
 // claimed, claims them beside its first workgroup and merges its bitmap.
 // Nobody waits for anybody; which workgroup traces a particle changes nothing
-// in the results.  25 wells, 1,000 particles, 20 years, 400 x 400 nodes, one
-// realization a workgroup -> shared: FP64 1 realization 3.1 -> 0.9 ms, 100
-// 8.4 -> 3.6, 1,000 19-42 (three draws) -> 14-21, 10,000 116 -> 112; its
-// unconfined field 1,000 98-246 -> 70-122; FP32 1,000 6.7-17.6 -> 4.8-7.6.
+// in the results.  25 wells, 1,000 particles, 20 years, 400 x 400 nodes, a
+// workgroup a realization -> shared: FP64 1 realization 3.0 -> 0.9 ms, 100 7.4 ->
+// 3.4, 1,000 17.5-41.4 (three draws) -> 13.9-22.3, 10,000 114.3 -> 111.8; its
+// unconfined field 1,000 97-244 -> 70-122; FP32 1,000 6.5-18.7 -> 4.5-7.3 (the
+// first with the wells as records in LDS).
 // kShareLeast: fewer particles are left to the lanes that are already there
 // (16 against 64 and 160: 2,000 realizations of 300 particles 12.3 ms against
 // 12.8, the others alike).

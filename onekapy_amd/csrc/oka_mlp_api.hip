@@ -501,8 +501,8 @@ int oka_mlp_train(oka_mlp *M, int64_t nsamples, const float *x, const uint8_t *m
         TRY(ensure(c, kSlotMlpLoss, sizeof(double) * nsteps, &dl));
         HIPCHK(c, launch_zero_f64((double *)dl, nsteps, c->stream));
     }
-    // Training steps (forward, backward, Adam with the BF16 refresh: 10
-    // launches each) are captured kStepsPerGraph at a time as a HIP graph and
+    // Training steps (forward, backward, Adam with the BF16 refresh: 9
+    // or 10 launches each) are captured kStepsPerGraph at a time as a HIP graph and
     // replayed; the step-dependent values (batch rows, loss slot, Adam step)
     // come from the device counters M->dstate, which each step's first and
     // last kernels advance.

@@ -250,9 +250,10 @@ int oka_trace_chronicle(oka_ctx *ctx, const oka_site *site, int32_t nreal, const
  * memory -- code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc -- this is oka_trace_chronicle with the same arguments and
  * results, whose scratch memory (statistics accumulators, the whole-grid
- * epoch, and the HBM bitmaps of grids too large for LDS) is a device array of
- * OKA_NOALLOC_SCRATCH_BYTES inside the library, which each GPU holds from the
- * library's first context on it until the process ends.  It calls no
+ * epoch, the FP32 wells' places, and the HBM bitmaps of grids too large for
+ * LDS) is a device array of OKA_NOALLOC_SCRATCH_BYTES and the places' 80 KiB
+ * inside the library, which each GPU holds from the library's first context on
+ * it until the process ends.  It calls no
  * allocator.  Restrictions:
  *   - flags must include OKA_PTR_DEVICE: every array argument (site->wells_xy,
  *     opts->start_xy and epochs included) is device memory;
